@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../host/amg_setup.hpp"
+#include "amg_dense.hpp"
 #include "la_kernels.hpp"
 
 namespace nodals {
@@ -118,6 +119,8 @@ class DevAmg {
     // same order as in the original numbering and results are identical.
     // perm[l][new] = original row; empty = not renumbered.
     std::vector<std::vector<int>> perm(nl), inv(nl);
+    dense_ = denseLevel(H, o);
+    std::vector<DenseSetupLevel> D(nl);
     for (std::size_t l = 0; l < nl; ++l) {
       const CsrD& A = H.A[l];
       Level& Lv = L_[l];
@@ -167,11 +170,30 @@ class DevAmg {
       for (DBuf<TV>* v : {&Lv.b, &Lv.x, &Lv.r, &Lv.tmp, &Lv.corr}) v->alloc((std::size_t)A.n);
       Lv.x.upload(std::vector<TV>((std::size_t)A.n, TV(1)));
       Lv.lambda = l < H.levelLambda.size() ? H.levelLambda[l] : 1.0;
+      if ((int)l >= dense_) {
+        D[l].n = A.n;
+        D[l].row.upload(r32);
+        D[l].col.upload(c32);
+        D[l].val.upload(v64);
+        D[l].diag.upload(d64);
+        D[l].l1.upload(l1);
+        D[l].lambda = Lv.lambda;
+        D[l].colorOff = Lv.color.off;
+      }
     }
     static const std::vector<int> none;
-    for (std::size_t l = 0; l < nl; ++l) uploadTransfer(H.P[l], P_[l], l > 0 ? inv[l - 1] : none, inv[l]);
+    for (std::size_t l = 0; l < nl; ++l)
+      uploadTransfer(H.P[l], P_[l], l > 0 ? inv[l - 1] : none, inv[l], (int)l > dense_ ? &D[l] : nullptr);
     termN_ = H.terminalN;
-    tinv_.upload(castVec(H.terminalInv));
+    {
+      const int ld = denseLd(termN_);
+      std::vector<TV> t((std::size_t)termN_ * ld, TV(0));
+      for (int i = 0; i < termN_; ++i)
+        for (int j = 0; j < termN_; ++j)
+          t[(std::size_t)i * ld + j] = (TV)H.terminalInv[(std::size_t)i * termN_ + j];
+      tinv_.upload(t);
+    }
+    if (dense_ < (int)nl - 1) buildDense(H, D);
     for (DBuf<TV>* v : {&fr_, &ftmp_, &fcorr_}) v->alloc((std::size_t)fineN);
     if (opt_.kind == "mcgs") {
       require(fineColoring != nullptr, "MCGS smoother requires a fine coloring", kErrInternal);
@@ -258,7 +280,7 @@ class DevAmg {
   // fine rows ascend) and relabelled afterwards, so its sums keep the
   // original order too.
   static void uploadTransfer(const Transfer& P, Xfer& X, const std::vector<int>& invF,
-                             const std::vector<int>& invC) {
+                             const std::vector<int>& invC, DenseSetupLevel* D) {
     X.nFine = P.nFine;
     X.nCoarse = P.nCoarse;
     auto relF = [&](int i) { return invF.empty() ? i : invF[(std::size_t)i]; };
@@ -316,7 +338,154 @@ class DevAmg {
     X.trow.upload(tr2);
     X.tcol.upload(tc2);
     X.tval.upload(castVec(tv2));
+    if (D) {  // FP64 copies, kept with the coarse side's level
+      D->prow.upload(pr);
+      D->pcol.upload(pc);
+      D->pval.upload(pv);
+      D->trow.upload(tr2);
+      D->tcol.upload(tc2);
+      D->tval.upload(tv2);
+    }
     X.lanesT = lanesFor(P.nCoarse ? (double)tc.size() / P.nCoarse : 1.0, P.nCoarse);
+  }
+
+  // Coarsest-first level from which the cycle is one dense product: the
+  // finest level whose product (n^2 values at 4.5 TB/s, 3 us of launch) costs
+  // less than the launches it replaces (2.2 us each: with MCGS two smoothing
+  // calls of a pass per colour, with the others their vector passes and
+  // residuals; about five more per level for transfers and residuals; the
+  // fused Jacobi cycle has four in all).  At most kDenseRows rows, 0.65 GB in
+  // FP64.  nl - 1, the terminal level, when no other pays.
+  static constexpr int kDenseRows = 9000;
+  int denseLevel(const AmgHierarchy& H, const SmootherOptions& o) const {
+    const int nl = (int)H.A.size();
+    double below = 3.0;  // us of the cycle below the level: the terminal product
+    int best = nl - 1;
+    for (int l = nl - 2; l >= 0; --l) {
+      const CsrD& A = H.A[(std::size_t)l];
+      if (A.n > kDenseRows) break;
+      double launches = 5.0;
+      if (o.kind == "mcgs") {
+        const Coloring C = greedyColoring(A.n, A.row.data(), A.col.data());
+        launches += 2.0 * o.mcgsCoarseSweeps * C.ncolors * (o.mcgsOrder == "symmetric" ? 2.0 : 1.0);
+      } else if (o.kind == "cheb2") {
+        launches += 2.0 * (1.0 + 2.0 * (o.chebDegree - 1)) + 2.0;
+      } else if (!fusedJacobi()) {
+        launches += 2.0 * (1.0 + 2.0 * (o.jacobiCoarseSweeps - 1)) + 2.0;
+      }
+      below += 2.2 * launches;
+      const double product = 3.0 + (double)A.n * denseLd(A.n) * sizeof(TV) / 4.5e6;
+      if (product < below) best = l;
+    }
+    return best;
+  }
+
+  // Sets denseT_ to the cycle from level dense_ down, column block by column
+  // block in FP64.
+  void buildDense(const AmgHierarchy& H, std::vector<DenseSetupLevel>& D) {
+    const int nl = (int)D.size(), n = D[(std::size_t)dense_].n, ld = denseLd(n);
+    const int block = std::min(n, 1024);
+    hipStream_t s = nullptr;
+    NODALS_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    try {
+      denseT_.alloc((std::size_t)n * ld);
+      fill<TV>(s, (long long)n * ld, denseT_.data(), TV(0));
+      for (int l = dense_; l < nl; ++l) {
+        DenseSetupLevel& L = D[(std::size_t)l];
+        for (DBuf<double>* v : {&L.b, &L.x, &L.r, &L.corr}) v->alloc((std::size_t)L.n * block);
+      }
+      DBuf<double> tinv;
+      tinv.upload(H.terminalInv);
+      DenseSetupLevel& T = D[(std::size_t)dense_];
+      for (int c0 = 0; c0 < n; c0 += block) {
+        const int m = std::min(block, n - c0);
+        const dim3 grid(n, (m + 255) / 256);
+        hipLaunchKernelGGL(k_cols_unit, grid, 256, 0, s, m, c0, T.b.data());
+        NODALS_LAUNCHED();
+        colsCycle(s, D, dense_, m, tinv);
+        hipLaunchKernelGGL(k_cols_store<TV>, grid, 256, 0, s, m, c0, ld, T.x.data(), denseT_.data());
+        NODALS_LAUNCHED();
+      }
+      NODALS_HIP(hipStreamSynchronize(s));
+      sweepScratch_.release();
+    } catch (...) {
+      (void)hipStreamSynchronize(s);
+      (void)hipStreamDestroy(s);
+      throw;
+    }
+    NODALS_HIP(hipStreamDestroy(s));
+  }
+
+  // vcycle() on m columns: D[l].x from D[l].b.
+  void colsCycle(hipStream_t s, std::vector<DenseSetupLevel>& D, int l, int m, const DBuf<double>& tinv) {
+    DenseSetupLevel& A = D[(std::size_t)l];
+    const dim3 grid(A.n, (m + 255) / 256);
+    if (l == (int)D.size() - 1) {
+      hipLaunchKernelGGL(k_cols_dense, grid, 256, 0, s, A.n, m, tinv.data(), A.b.data(), A.x.data());
+      NODALS_LAUNCHED();
+      return;
+    }
+    DenseSetupLevel& C = D[(std::size_t)l + 1];
+    colsSmooth(s, A, m, A.b.data(), A.x.data());
+    hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), A.x.data(),
+                       A.b.data(), A.r.data());
+    hipLaunchKernelGGL((k_cols_spmv<0>), dim3(C.n, grid.y), 256, 0, s, m, C.trow.data(), C.tcol.data(), C.tval.data(),
+                       A.r.data(), nullptr, C.b.data());
+    NODALS_LAUNCHED();
+    colsCycle(s, D, l + 1, m, tinv);
+    hipLaunchKernelGGL((k_cols_spmv<2>), grid, 256, 0, s, m, C.prow.data(), C.pcol.data(), C.pval.data(), C.x.data(),
+                       nullptr, A.x.data());
+    hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), A.x.data(),
+                       A.b.data(), A.r.data());
+    NODALS_LAUNCHED();
+    // the post-smoothing reads A.r and needs a residual of its own: A.b is
+    // not read again
+    colsSmooth(s, A, m, A.r.data(), A.corr.data());
+    hipLaunchKernelGGL(k_cols_axpy, grid, 256, 0, s, m, A.corr.data(), A.x.data());
+    NODALS_LAUNCHED();
+  }
+
+  // smooth() on m columns from x = 0.
+  void colsSmooth(hipStream_t s, DenseSetupLevel& A, int m, const double* b, double* x) {
+    const dim3 grid(A.n, (m + 255) / 256);
+    if (opt_.kind == "mcgs") {
+      fill<double>(s, (long long)A.n * m, x, 0.0);
+      const int nc = (int)A.colorOff.size() - 1;
+      auto pass = [&](bool reverse) {
+        for (int q = 0; q < nc; ++q) {
+          const int c = reverse ? nc - 1 - q : q;
+          const int begin = A.colorOff[(std::size_t)c], count = A.colorOff[(std::size_t)c + 1] - begin;
+          if (count <= 0) continue;
+          hipLaunchKernelGGL(k_cols_gs, dim3(count, grid.y), 256, 0, s, m, begin, A.row.data(), A.col.data(),
+                             A.val.data(), A.diag.data(), b, x, opt_.mcgsOmega);
+          NODALS_LAUNCHED();
+        }
+      };
+      for (int sw = 0; sw < opt_.mcgsCoarseSweeps; ++sw) {
+        if (opt_.mcgsOrder != "backward") pass(false);
+        if (opt_.mcgsOrder != "forward") pass(true);
+      }
+      return;
+    }
+    const bool cheb = opt_.kind == "cheb2";
+    const double lo = opt_.lambdaLowFraction * A.lambda;
+    require(!cheb || (A.lambda > lo && lo > 0), "Chebyshev interval invalid");
+    const int steps = cheb ? opt_.chebDegree : opt_.jacobiCoarseSweeps;
+    const double* den = opt_.kind == "l1jacobi" ? A.l1.data() : A.diag.data();
+    DBuf<double>& t = sweepScratch_;
+    if (steps > 1 && t.size() < (std::size_t)A.n * m) t.alloc((std::size_t)A.n * m);
+    for (int k = 0; k < steps; ++k) {
+      const double w = cheb ? 1.0 / chebRoot(A.lambda, lo, k, opt_.chebDegree) : opt_.jacobiOmega;
+      const double* r = b;
+      if (k > 0) {
+        hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), x, b,
+                           t.data());
+        NODALS_LAUNCHED();
+        r = t.data();
+      }
+      hipLaunchKernelGGL(k_cols_jacobi, grid, 256, 0, s, m, w, r, den, x, k > 0 ? 1 : 0);
+      NODALS_LAUNCHED();
+    }
   }
 
   void restrictTo(hipStream_t s, const Xfer& X, const TV* f, TV* c) {
@@ -411,9 +580,8 @@ class DevAmg {
 
   void vcycle(hipStream_t s, int l, const TV* b, TV* x) {
     Level& A = L_[(std::size_t)l];
-    if (l == (int)L_.size() - 1) {
-      hipLaunchKernelGGL(k_dense_mv<TV>, blocksFor((long long)A.n * 64), 256, 0, s, A.n, tinv_.data(), b, x);
-      NODALS_LAUNCHED();
+    if (l == dense_) {  // the terminal level, or the whole sub-cycle in one product
+      denseMv<TV>(s, A.n, dense_ == (int)L_.size() - 1 ? tinv_.data() : denseT_.data(), b, x);
       return;
     }
     if (fusedJacobi()) {
@@ -458,8 +626,9 @@ class DevAmg {
   DevColoring<TV> fineColor_;
   std::vector<Level> L_;
   std::vector<Xfer> P_;
-  DBuf<TV> tinv_;
-  int termN_ = 0;
+  DBuf<TV> tinv_, denseT_;
+  DBuf<double> sweepScratch_;  // dense set-up only
+  int termN_ = 0, dense_ = 0;
   DBuf<TV> fr_, ftmp_, fcorr_;
   GraphCache graph_;
   GraphSet wide_;

@@ -434,21 +434,6 @@ __global__ void __launch_bounds__(1024) k_mcgs_level_wg(int n, const int* __rest
   for (int i = threadIdx.x; i < n; i += blockDim.x) x[i] = xs[i];
 }
 
-// x = T b for a dense row-major n x n matrix (terminal AMG level).
-template <class TV>
-__global__ void __launch_bounds__(256) k_dense_mv(int n, const TV* __restrict__ T, const TV* __restrict__ b,
-                                                  TV* __restrict__ x) {
-  const int gid = blockIdx.x * 256 + threadIdx.x;
-  const int r = gid >> 6;
-  const int lane = gid & 63;
-  if (r >= n) return;
-  TV s = 0;
-  const TV* tr = T + (long long)r * n;
-  for (int j = lane; j < n; j += 64) s += tr[j] * b[j];
-  s = groupSum(s, 64);
-  if (lane == 0) x[r] = s;
-}
-
 template <class T>
 __global__ void k_diag_gather(int n, const int* __restrict__ diagPos, const T* __restrict__ val, T* __restrict__ d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
