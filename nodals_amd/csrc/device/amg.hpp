@@ -17,6 +17,7 @@
 
 #include "../host/amg_setup.hpp"
 #include "amg_dense.hpp"
+#include "gs_ell.hpp"
 #include "la_kernels.hpp"
 
 namespace nodals {
@@ -31,29 +32,13 @@ struct SmootherOptions {
   double mcgsOmega = 1.0;
   int mcgsFineSweeps = 1, mcgsCoarseSweeps = 1;
   std::string mcgsOrder = "symmetric";  // forward | backward | symmetric
-  // Coarse levels with at most this many nonzeros (and vectors that fit
-  // kFuseLdsBytes of LDS) run each MCGS smoothing call as one workgroup
-  // (k_mcgs_level_wg) instead of one launch per colour; 0 turns it off.
-  // One CU streams a level's matrix once per colour pass: on the 207k helix's
-  // CF hierarchy the 108k-nonzero level gains and the 873k-nonzero level
-  // loses against launches spread over the chip.
-  long long mcgsFuseNnz = 250000;
 };
-
-// LDS of the fused level smoother: iterate, right-hand side, diagonal and
-// row pointers.
-constexpr std::size_t kFuseLdsBytes = 96 * 1024;
-template <class TV>
-constexpr std::size_t fuseLdsBytes(int n) {
-  return (std::size_t)n * (3 * sizeof(TV) + sizeof(int)) + sizeof(int);
-}
 
 // View of the finest operator, owned elsewhere (refreshed each SIMPLE step).
 template <class TF, class TV>
 struct FineView {
   int n = 0;
   int lanes = 16;
-  double meanRow = 8.0;  // nonzeros per row (lanes of the per-colour passes)
   const int* row = nullptr;
   const int* col = nullptr;
   const TF* val = nullptr;
@@ -81,18 +66,39 @@ struct DevColoring {
   const int* rowList() const { return contiguous ? nullptr : rows.data(); }
 };
 
+// The slots an MCGS smoothing call reads: the half that a pass from x = 0
+// needs, the other half for symmetric sweeps, and every off-diagonal entry
+// for the later sweeps of a one-directional order.
+template <class TM>
+struct GsOperator {
+  GsSlots<TM> lower, upper, all;
+  template <class TI>
+  void build(int ncolors, const std::vector<int>& off, const int* rows, int n, const TI* row, const int* col,
+             const std::string& order, int sweeps, const TM* csr) {
+    std::vector<int> colorOf((std::size_t)n, 0);
+    for (int c = 0; c < ncolors; ++c)
+      for (int q = off[(std::size_t)c]; q < off[(std::size_t)c + 1]; ++q) colorOf[(std::size_t)(rows ? rows[q] : q)] = c;
+    if (order != "backward") lower.upload(gsLayout(ncolors, off, rows, colorOf, row, col, GsHalf::lower), csr);
+    if (order != "forward") upper.upload(gsLayout(ncolors, off, rows, colorOf, row, col, GsHalf::upper), csr);
+    if (order != "symmetric" && sweeps > 1)
+      all.upload(gsLayout(ncolors, off, rows, colorOf, row, col, GsHalf::all), csr);
+  }
+  template <class TI>
+  void fill(hipStream_t s, const TI* csr) {
+    for (GsSlots<TM>* g : {&lower, &upper, &all}) g->fill(s, csr);
+  }
+};
+
 template <class TF, class TV>
 class DevAmg {
  public:
   struct Level {
     int n = 0, lanes = 8;
-    double meanRow = 1.0;
     DBuf<int> row, col;
     DBuf<TV> val, diag, l1, b, x, r, tmp, corr;
     double lambda = 1.0;
     DevColoring<TV> color;
-    bool fused = false;          // MCGS smoothing in one workgroup
-    DBuf<int> colorOff, colorLanes;
+    GsOperator<TV> gs;
   };
   struct Xfer {
     int nFine = 0, nCoarse = 0, lanesP = 8, lanesT = 8;
@@ -125,22 +131,13 @@ class DevAmg {
       const CsrD& A = H.A[l];
       Level& Lv = L_[l];
       Lv.n = A.n;
-      Lv.meanRow = A.n ? (double)A.col.size() / A.n : 1.0;
-      Lv.lanes = lanesFor(Lv.meanRow, A.n);
+      Lv.lanes = lanesFor(A.n ? (double)A.col.size() / A.n : 1.0, A.n);
       if (opt_.kind == "mcgs" && l + 1 < nl) {
         const Coloring C = greedyColoring(A.n, A.row.data(), A.col.data());
         perm[l].assign(C.rows.begin(), C.rows.end());
         inv[l].assign((std::size_t)A.n, 0);
         for (int i = 0; i < A.n; ++i) inv[l][(std::size_t)perm[l][(std::size_t)i]] = i;
         Lv.color.uploadContiguous(C);
-        if (o.mcgsFuseNnz > 0 && (long long)A.col.size() <= o.mcgsFuseNnz && fuseLdsBytes<TV>(A.n) <= kFuseLdsBytes) {
-          std::vector<int> lanes((std::size_t)C.ncolors);
-          for (int c = 0; c < C.ncolors; ++c)
-            lanes[(std::size_t)c] = lanesFor(Lv.meanRow, C.offset[(std::size_t)c + 1] - C.offset[(std::size_t)c]);
-          Lv.colorOff.upload(C.offset);
-          Lv.colorLanes.upload(lanes);
-          Lv.fused = true;
-        }
       }
       const std::vector<int>& pm = perm[l];
       const std::vector<int>& iv = inv[l];
@@ -165,6 +162,10 @@ class DevAmg {
       Lv.row.upload(r32);
       Lv.col.upload(c32);
       Lv.val.upload(castVec(v64));
+      if (opt_.kind == "mcgs" && (int)l < dense_) {
+        Lv.gs.build(Lv.color.ncolors, Lv.color.off, nullptr, A.n, r32.data(), c32.data(), opt_.mcgsOrder,
+                    opt_.mcgsCoarseSweeps, castVec(v64).data());
+      }
       Lv.diag.upload(castVec(d64));
       Lv.l1.upload(castVec(l1));
       for (DBuf<TV>* v : {&Lv.b, &Lv.x, &Lv.r, &Lv.tmp, &Lv.corr}) v->alloc((std::size_t)A.n);
@@ -198,10 +199,19 @@ class DevAmg {
     if (opt_.kind == "mcgs") {
       require(fineColoring != nullptr, "MCGS smoother requires a fine coloring", kErrInternal);
       fineColor_.upload(*fineColoring);
+      for (DBuf<TV>* v : {&gsA_, &gsB_}) v->alloc((std::size_t)fineN);
     }
   }
 
-  void setFine(const FineView<TF, TV>& v) { fine_ = v; }
+  // The finest operator, with its pattern on the host (row[n + 1], col).  Call
+  // fineChanged() whenever its values have changed.
+  void setFine(const FineView<TF, TV>& v, const int* hostRow, const int* hostCol, const Coloring* C) {
+    fine_ = v;
+    if (opt_.kind == "mcgs")
+      fineGs_.build(C->ncolors, C->offset, C->rows.data(), v.n, hostRow, hostCol, opt_.mcgsOrder, opt_.mcgsFineSweeps,
+                    nullptr);
+  }
+  void fineChanged(hipStream_t s) { fineGs_.fill(s, fine_.val); }
   // tmp = A_l x on explicit level l (measurement of the coarse SpMV).
   void levelSpmv(hipStream_t s, int l) {
     Level& A = L_[(std::size_t)l];
@@ -501,11 +511,11 @@ class DevAmg {
     return centre - radius * std::cos(pi * (2.0 * k + 1.0) / (2.0 * degree));
   }
 
-  // Generic smoother on an operator (row, col, val, diag, l1) from x = 0.
+  // Jacobi and Chebyshev smoothing of an operator (row, col, val, diag, l1)
+  // from x = 0; r is scratch.
   template <class TM>
-  void smooth(hipStream_t s, int n, int lanes, double meanRow, const int* row, const int* col, const TM* val, const TV* diag,
-              const TV* l1, const DevColoring<TV>* color, double lambda, int jacobiSweeps, int mcgsSweeps,
-              const TV* b, TV* x, TV* tmp, TV* r) {
+  void smooth(hipStream_t s, int n, int lanes, const int* row, const int* col, const TM* val, const TV* diag,
+              const TV* l1, double lambda, int jacobiSweeps, const TV* b, TV* x, TV* r) {
     const int grid = blocksFor(n);
     if (opt_.kind == "jacobi" || opt_.kind == "l1jacobi") {
       const TV* den = opt_.kind == "l1jacobi" ? l1 : diag;
@@ -528,54 +538,53 @@ class DevAmg {
                            diag, x);
         NODALS_LAUNCHED();
       }
-    } else if (opt_.kind == "mcgs") {
-      fill<TV>(s, n, x, TV(0));
-      for (int sw = 0; sw < mcgsSweeps; ++sw) {
-        if (opt_.mcgsOrder == "forward" || opt_.mcgsOrder == "symmetric")
-          colorPass(s, meanRow, row, col, val, diag, b, x, *color, false);
-        if (opt_.mcgsOrder == "backward" || opt_.mcgsOrder == "symmetric")
-          colorPass(s, meanRow, row, col, val, diag, b, x, *color, true);
-      }
     } else {
       fail("unknown AMG smoother " + opt_.kind);
     }
-    (void)tmp;
   }
 
+  // MCGS smoothing from x = 0 (no pass reads an entry of x that an earlier
+  // one has not written, so x is not cleared).  A symmetric sweep's passes
+  // keep the row sum of the half that does not change until the next pass.
   template <class TM>
-  void colorPass(hipStream_t s, double meanRow, const int* row, const int* col, const TM* val, const TV* diag, const TV* b,
-                 TV* x, const DevColoring<TV>& C, bool reverse) {
-    for (int q = 0; q < C.ncolors; ++q) {
-      const int c = reverse ? C.ncolors - 1 - q : q;
-      const int begin = C.off[(std::size_t)c], count = C.off[(std::size_t)c + 1] - begin;
-      mcgsColor<TM, TV>(s, lanesFor(meanRow, count), begin, count, C.rowList(), row, col, val, diag, b, x,
-                        opt_.mcgsOmega);
+  void mcgsSmooth(hipStream_t s, const GsOperator<TM>& G, const DevColoring<TV>& C, int sweeps, const TV* diag,
+                  const TV* b, TV* x) {
+    auto pass = [&](const GsSlots<TM>& S, bool reverse, const TV* other, TV* part, bool zero) {
+      for (int q = 0; q < C.ncolors; ++q) {
+        const int c = reverse ? C.ncolors - 1 - q : q;
+        const int begin = C.off[(std::size_t)c], count = C.off[(std::size_t)c + 1] - begin;
+        gsColour<TM, TV>(s, S.colour[(std::size_t)c], begin, count, C.rowList(), S.col.data(), S.val.data(), diag, b, x,
+                         other, part, zero, opt_.mcgsOmega);
+      }
+    };
+    const bool back = opt_.mcgsOrder == "backward";
+    for (int sw = 0; sw < sweeps; ++sw) {
+      const bool first = sw == 0, last = sw == sweeps - 1;
+      if (opt_.mcgsOrder == "symmetric") {
+        pass(G.lower, false, first ? nullptr : gsB_.data(), gsA_.data(), first);
+        pass(G.upper, true, gsA_.data(), last ? nullptr : gsB_.data(), false);
+      } else {
+        pass(first ? (back ? G.upper : G.lower) : G.all, back, nullptr, nullptr, first);
+      }
     }
   }
 
   void smoothFine(hipStream_t s, const TV* b, TV* x) {
-    smooth<TF>(s, fine_.n, fine_.lanes, fine_.meanRow, fine_.row, fine_.col, fine_.val, fine_.diag, fine_.l1, &fineColor_,
-               fineLambda_, opt_.jacobiFineSweeps, opt_.mcgsFineSweeps, b, x, ftmp_.data(), ftmp_.data());
+    if (opt_.kind == "mcgs") {
+      mcgsSmooth<TF>(s, fineGs_, fineColor_, opt_.mcgsFineSweeps, fine_.diag, b, x);
+      return;
+    }
+    smooth<TF>(s, fine_.n, fine_.lanes, fine_.row, fine_.col, fine_.val, fine_.diag, fine_.l1, fineLambda_,
+               opt_.jacobiFineSweeps, b, x, ftmp_.data());
   }
 
   void smoothLevel(hipStream_t s, Level& A, const TV* b, TV* x) {
-    if (A.fused) {
-      const int order = opt_.mcgsOrder == "forward" ? 0 : opt_.mcgsOrder == "backward" ? 1 : 2;
-      const std::size_t lds = fuseLdsBytes<TV>(A.n);
-      static const bool attr = [] {
-        NODALS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mcgs_level_wg<TV, TV>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFuseLdsBytes));
-        return true;
-      }();
-      (void)attr;
-      hipLaunchKernelGGL((k_mcgs_level_wg<TV, TV>), 1, 1024, lds, s, A.n, A.row.data(), A.col.data(), A.val.data(),
-                         A.diag.data(), b, x, A.color.ncolors, A.colorOff.data(), A.colorLanes.data(),
-                         opt_.mcgsCoarseSweeps, order, opt_.mcgsOmega);
-      NODALS_LAUNCHED();
+    if (opt_.kind == "mcgs") {
+      mcgsSmooth<TV>(s, A.gs, A.color, opt_.mcgsCoarseSweeps, A.diag.data(), b, x);
       return;
     }
-    smooth<TV>(s, A.n, A.lanes, A.meanRow, A.row.data(), A.col.data(), A.val.data(), A.diag.data(), A.l1.data(), &A.color,
-               A.lambda, opt_.jacobiCoarseSweeps, opt_.mcgsCoarseSweeps, b, x, A.tmp.data(), A.tmp.data());
+    smooth<TV>(s, A.n, A.lanes, A.row.data(), A.col.data(), A.val.data(), A.diag.data(), A.l1.data(), A.lambda,
+               opt_.jacobiCoarseSweeps, b, x, A.tmp.data());
   }
 
   void vcycle(hipStream_t s, int l, const TV* b, TV* x) {
@@ -624,6 +633,8 @@ class DevAmg {
   double fineLambda_ = 1.0;
   FineView<TF, TV> fine_;
   DevColoring<TV> fineColor_;
+  GsOperator<TF> fineGs_;
+  DBuf<TV> gsA_, gsB_;  // row sums kept between the passes of a symmetric sweep
   std::vector<Level> L_;
   std::vector<Xfer> P_;
   DBuf<TV> tinv_, denseT_;

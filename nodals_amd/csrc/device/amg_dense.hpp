@@ -70,6 +70,22 @@ void denseMv(hipStream_t s, int n, const TV* T, const TV* b, TV* x) {
   NODALS_LAUNCHED();
 }
 
+// Sum over a row of val * x[col][c] with eight gathers in flight (the row's
+// columns and values are uniform over the block); column `skip` is left out.
+__device__ __forceinline__ double colsRow(int k, int e, const int* __restrict__ col, const double* __restrict__ val,
+                                          const double* x, int m, int c, int skip) {
+  double s = 0.0;
+  for (; k < e; k += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = x[(long long)col[min(k + u, e - 1)] * m + c];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (k + u < e && col[k + u] != skip) s += val[k + u] * v[u];
+  }
+  return s;
+}
+
 // The cycle on blocks of m columns, row-major: entry (i, c) at i*m + c.  One
 // thread an entry; blockIdx.x is the row, so every column reads the row's
 // values together.
@@ -82,8 +98,7 @@ static __global__ void __launch_bounds__(256) k_cols_spmv(int m, const int* __re
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= m) return;
   const long long o = (long long)blockIdx.x * m + c;
-  double s = 0.0;
-  for (int k = row[blockIdx.x]; k < row[blockIdx.x + 1]; ++k) s += val[k] * x[(long long)col[k] * m + c];
+  const double s = colsRow(row[blockIdx.x], row[blockIdx.x + 1], col, val, x, m, c, -1);
   y[o] = MODE == 0 ? s : MODE == 1 ? b[o] - s : y[o] + s;
 }
 // x = (add ? x : 0) + omega r / d
@@ -102,9 +117,7 @@ static __global__ void __launch_bounds__(256) k_cols_gs(int m, int begin, const 
                                                         double* x, double omega) {
   const int c = blockIdx.y * 256 + threadIdx.x, i = begin + blockIdx.x;
   if (c >= m) return;
-  double s = 0.0;
-  for (int k = row[i]; k < row[i + 1]; ++k)
-    if (col[k] != i) s += val[k] * x[(long long)col[k] * m + c];
+  const double s = colsRow(row[i], row[i + 1], col, val, x, m, c, i);
   const long long o = (long long)i * m + c;
   const double old = x[o];
   x[o] = old + omega * ((b[o] - s) / d[i] - old);
@@ -115,6 +128,7 @@ static __global__ void __launch_bounds__(256) k_cols_dense(int n, int m, const d
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= m) return;
   double s = 0.0;
+#pragma unroll 8
   for (int j = 0; j < n; ++j) s += T[(long long)blockIdx.x * n + j] * b[(long long)j * m + c];
   x[(long long)blockIdx.x * m + c] = s;
 }

@@ -20,33 +20,41 @@
 //
 // Measured on gfx950, microseconds per colour pass in a replayed graph, CSR
 // launches against these (a chain of empty launches takes 1.9):
-//   207k-cell P0 Schur operator, 35 colours, 68 nonzeros a row: 5.4 -> 3.6
-//   69k-row CF level, 39 colours, 74 a row: 4.6 -> 3.1
+//   207k-cell P0 Schur operator, 35 colours, 68 nonzeros a row: 5.4 -> 3.5
+//   69k-row CF level, 39 colours, 74 a row: 4.6 -> 2.9
 //   8.5k-row CF level, 47 colours, 102 a row: 3.8 -> 2.3
-//   64^3 P1 Laplacian, 8 colours, 15 a row: 6.5 -> 4.0
+//   64^3 P1 Laplacian, 8 colours, 15 a row: 6.5 -> 3.9
+//   7.5k-row k-omega vertex operator, 10 colours, 14 a row: 3.7 -> 2.5
+// Half of that is the reduction over lanes in registers, the exact slot count
+// as a template argument and the missing row pointers; a fixed count of eight
+// with predicated slots costs 0.3-0.4 us a pass more.
 #pragma once
 
 #include <algorithm>
+#include <thread>
 #include <vector>
 
+#include "../host/h8_setup.hpp"
 #include "la_kernels.hpp"
 
 namespace nodals {
 namespace dev {
 
-constexpr int kGsUnroll = 8;  // slots a lane loads before it gathers
+constexpr int kGsUnroll = 8;  // most slots a lane loads before it gathers
 
 // Which off-diagonal entries of a row a GsSlots holds.
 enum class GsHalf { lower, upper, all };
 
-// Host layout of one colour's slots: first tile, lanes a row, slots a lane.
+// Host layout of one colour's slots: first tile, lanes a row, slots a lane
+// (at most kGsUnroll, or a multiple of it).
 struct GsColour {
   int tile = 0, L = 1, U = 1;
 };
 
 // Lanes a row for `count` rows of at most `width` entries: the fewest that
-// leave a lane at most kGsUnroll/2 slots, widened while the colour is too small to
-// give every SIMD a wavefront (2^16 threads) and a lane still holds two.
+// leave a lane at most kGsUnroll/2 slots, widened while the colour is too
+// small to give every SIMD a wavefront (2^16 threads) and a lane still holds
+// two: within 4% of the best of 1..64 lanes on every operator above.
 inline int gsLanes(int width, int count) {
   int L = 1;
   while (L < 64 && (width > L * (kGsUnroll / 2) || ((long long)count * L < (1 << 16) && width > 2 * L))) L *= 2;
@@ -55,14 +63,15 @@ inline int gsLanes(int width, int count) {
 
 // Tiled slots of the chosen half of a coloured CSR operator (rows of colour
 // c: rows[off[c]..off[c+1]), or those indices themselves when rows is null).
+// Colours are independent: they are counted, then filled, in parallel.
 struct GsLayout {
   std::vector<GsColour> colour;
-  std::vector<int> col, src;  // column (pad where unused), CSR position (-1 where unused)
+  std::vector<int> col, src;  // column (-1 where unused), CSR position (-1 where unused)
 };
 
 template <class TI>
 GsLayout gsLayout(int ncolors, const std::vector<int>& off, const int* rows, const std::vector<int>& colorOf,
-                  const TI* row, const int* col, GsHalf half, int pad = -1, int forceL = 0, int minU = 1) {
+                  const TI* row, const int* col, GsHalf half) {
   GsLayout G;
   G.colour.resize((std::size_t)ncolors);
   auto wanted = [&](int i, int j, int c) {
@@ -70,8 +79,16 @@ GsLayout gsLayout(int ncolors, const std::vector<int>& off, const int* rows, con
     const int cj = colorOf[(std::size_t)j];
     return half == GsHalf::all || (half == GsHalf::lower ? cj < c : cj > c);
   };
-  for (int c = 0; c < ncolors; ++c) {
-    const int b = off[(std::size_t)c], n = off[(std::size_t)c + 1] - b;
+  auto eachColour = [&](auto&& body) {
+    const int nt = std::max(1, std::min(ncolors, off.back() < 4096 ? 1 : hostThreads(0)));
+    std::vector<std::thread> pool;
+    for (int t = 0; t < nt; ++t)
+      pool.emplace_back([&, t]() {
+        for (int c = t; c < ncolors; c += nt) body(c, off[(std::size_t)c], off[(std::size_t)c + 1] - off[(std::size_t)c]);
+      });
+    for (std::thread& th : pool) th.join();
+  };
+  eachColour([&](int c, int b, int n) {
     int width = 1;
     for (int q = 0; q < n; ++q) {
       const int i = rows ? rows[b + q] : b + q;
@@ -80,14 +97,23 @@ GsLayout gsLayout(int ncolors, const std::vector<int>& off, const int* rows, con
       width = std::max(width, w);
     }
     GsColour& C = G.colour[(std::size_t)c];
-    C.L = forceL > 0 ? forceL : gsLanes(width, n);
+    C.L = gsLanes(width, n);
     C.U = (width + C.L - 1) / C.L;
     if (C.U > kGsUnroll) C.U = (C.U + kGsUnroll - 1) / kGsUnroll * kGsUnroll;
-    C.U = std::max(C.U, minU);
-    C.tile = (int)(G.col.size() / 64);
-    const int per = 64 / C.L, tiles = (n + per - 1) / per;
-    G.col.resize(G.col.size() + (std::size_t)tiles * C.U * 64, pad);
-    G.src.resize(G.col.size(), -1);
+  });
+  long long tiles = 0;
+  for (int c = 0; c < ncolors; ++c) {
+    GsColour& C = G.colour[(std::size_t)c];
+    const int n = off[(std::size_t)c + 1] - off[(std::size_t)c], per = 64 / C.L;
+    C.tile = (int)tiles;
+    tiles += (long long)((n + per - 1) / per) * C.U;
+    require(tiles < (1ll << 31), "Gauss-Seidel slots too large for int32 tile indices");
+  }
+  G.col.assign((std::size_t)tiles * 64, -1);
+  G.src.assign((std::size_t)tiles * 64, -1);
+  eachColour([&](int c, int b, int n) {
+    const GsColour& C = G.colour[(std::size_t)c];
+    const int per = 64 / C.L;
     for (int q = 0; q < n; ++q) {
       const int i = rows ? rows[b + q] : b + q;
       const std::size_t at = ((std::size_t)C.tile + (std::size_t)(q / per) * C.U) * 64 + (std::size_t)(q % per) * C.L;
@@ -100,68 +126,18 @@ GsLayout gsLayout(int ncolors, const std::vector<int>& off, const int* rows, con
           ++w;
         }
     }
-  }
+  });
   return G;
 }
 
-// Sum over groups of L consecutive lanes (every lane gets it) with cross-lane
-// moves inside the registers: quad swaps, half-row and row mirrors (the
-// mirrored lanes hold equal partial sums already), then 16- and 32-lane swaps.
-template <int CTRL>
-__device__ __forceinline__ int dppMove(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ __forceinline__ float dppMove(float v) {
-  return __int_as_float(dppMove<CTRL>(__float_as_int(v)));
-}
-__device__ __forceinline__ double fromWords(unsigned lo, unsigned hi) {
-  return __longlong_as_double(((long long)(int)hi << 32) | lo);
-}
-template <int CTRL>
-__device__ __forceinline__ double dppMove(double v) {
-  const long long b = __double_as_longlong(v);
-  return fromWords((unsigned)dppMove<CTRL>((int)b), (unsigned)dppMove<CTRL>((int)(b >> 32)));
-}
-__device__ __forceinline__ float swapAdd16(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ double swapAdd16(double v) {
-  const long long b = __double_as_longlong(v);
-  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
-  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-  return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
-}
-__device__ __forceinline__ float swapAdd32(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ double swapAdd32(double v) {
-  const long long b = __double_as_longlong(v);
-  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
-  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-  return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
-}
-template <int L, class T>
-__device__ __forceinline__ T laneSum(T v) {
-  if constexpr (L >= 2) v += dppMove<0xB1>(v);   // quad_perm [1,0,3,2]
-  if constexpr (L >= 4) v += dppMove<0x4E>(v);   // quad_perm [2,3,0,1]
-  if constexpr (L >= 8) v += dppMove<0x141>(v);  // row_half_mirror
-  if constexpr (L >= 16) v += dppMove<0x140>(v);  // row_mirror
-  if constexpr (L >= 32) v = swapAdd16(v);
-  if constexpr (L >= 64) v = swapAdd32(v);
-  return v;
-}
-
 // Slot values gathered from the CSR values they mirror.
-template <class TM>
-__global__ void __launch_bounds__(256) k_gs_fill(long long n, const int* __restrict__ src, const TM* __restrict__ val,
-                                                 TM* __restrict__ out) {
+template <class TO, class TI>
+__global__ void __launch_bounds__(256) k_gs_fill(long long n, const int* __restrict__ src, const TI* __restrict__ val,
+                                                 TO* __restrict__ out) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const int s = src[i];
-  out[i] = s >= 0 ? val[s] : TM{};
+  out[i] = s >= 0 ? (TO)val[s] : TO{};
 }
 
 // One colour pass over rows crow[begin + q] (begin + q without a list), q <
@@ -255,95 +231,35 @@ void gsColour(hipStream_t s, const GsColour& C, int begin, int count, const int*
   }
 }
 
-// ---------------------------------------------------------------- one workgroup
-// A step of the one-workgroup sweep: rows [row0, row0 + count) of one colour
-// (the operator numbered in colour order), their first tile and slots a lane.
-struct GsStep {
-  int row0, count, tile, U;
+// Device slots of one half of an operator.
+template <class TM>
+struct GsSlots {
+  std::vector<GsColour> colour;
+  DBuf<int> col, src;
+  DBuf<TM> val;
+  // With the operator's values when they are fixed; otherwise fill() them.
+  void upload(const GsLayout& G, const TM* csr) {
+    colour = G.colour;
+    col.upload(G.col);
+    if (!csr) {
+      src.upload(G.src);
+      val.alloc(G.src.size());
+      return;
+    }
+    std::vector<TM> v(G.src.size(), TM{});
+    for (std::size_t k = 0; k < v.size(); ++k)
+      if (G.src[k] >= 0) v[k] = csr[G.src[k]];
+    val.upload(v);
+  }
+  // Values from the operator's CSR values.
+  template <class TI>
+  void fill(hipStream_t s, const TI* csr) {
+    const long long n = (long long)src.size();
+    if (n == 0) return;
+    hipLaunchKernelGGL((k_gs_fill<TM, TI>), blocksFor(n), 256, 0, s, n, src.data(), csr, val.data());
+    NODALS_LAUNCHED();
+  }
 };
-
-template <int U, class TM, class TV>
-struct GsRegs {
-  int c[U];
-  TM a[U];
-  TV b, inv, other;
-};
-
-template <int L, int U, class TM, class TV>
-__device__ __forceinline__ void gsLoad(const GsStep& st, const int* __restrict__ col, const TM* __restrict__ val,
-                                       const TV* __restrict__ inv, const TV* __restrict__ b, const TV* part,
-                                       GsRegs<U, TM, TV>& r) {
-  constexpr int per = 64 / L;
-  const int lane = threadIdx.x & 63, tiles = (st.count + per - 1) / per;
-  const int w = min((int)(threadIdx.x >> 6), tiles - 1);  // a wavefront without rows loads the last tile
-  const int q = w * per + lane / L, i = st.row0 + min(q, st.count - 1);
-  const int at = (st.tile + w * U) * 64 + lane;
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    r.c[u] = col[at + u * 64];
-    r.a[u] = val[at + u * 64];
-  }
-  r.b = b[i];
-  r.inv = inv[i];
-  r.other = part[i];
-}
-
-// Barrier that orders LDS only: global loads in flight stay in flight.
-__device__ __forceinline__ void ldsBarrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int L, int U, class TM, class TV>
-__device__ __forceinline__ void gsApply(const GsStep& st, const GsRegs<U, TM, TV>& r, TV* xs, TV* part, bool zero,
-                                        bool useOther, double omega) {
-  constexpr int per = 64 / L;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int q = w * per + lane / L, i = st.row0 + min(q, st.count - 1);
-  const TV old = zero ? TV(0) : xs[i];
-  TV v[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) v[u] = xs[r.c[u]];
-  TV s = 0;
-#pragma unroll
-  for (int u = 0; u < U; ++u) s += (TV)r.a[u] * v[u];
-  s = laneSum<L>(s);
-  if (lane % L == 0 && q < st.count) {
-    if (part) part[i] = s;
-    const TV t = useOther ? s + r.other : s;
-    xs[i] = old + (TV)omega * ((r.b - t) * r.inv - old);
-  }
-  ldsBarrier();
-}
-
-// One pass over ns steps (backwards when rev): the next step's slots are
-// loaded into registers before this one's gathers, so between two barriers
-// only LDS reads, the row sums and the update remain.
-template <int L, int U, class TM, class TV>
-__device__ __forceinline__ void gsPass(int ns, bool rev, const GsStep* __restrict__ step, const int* __restrict__ col,
-                                       const TM* __restrict__ val, const TV* __restrict__ inv,
-                                       const TV* __restrict__ b, TV* xs, const TV* other, bool useOther, TV* part,
-                                       bool zero, double omega) {
-  auto at = [&](int k) {
-    k = min(k, ns - 1);
-    return step[rev ? ns - 1 - k : k];
-  };
-  GsRegs<U, TM, TV> A, B;
-  GsStep s0 = at(0), s1 = at(1);
-  gsLoad<L>(s0, col, val, inv, b, other, A);
-  int k = 0;
-  for (; k + 1 < ns; k += 2) {
-    const GsStep s2 = at(k + 2), s3 = at(k + 3);
-    gsLoad<L>(s1, col, val, inv, b, other, B);
-    gsApply<L>(s0, A, xs, part, zero, useOther, omega);
-    gsLoad<L>(s2, col, val, inv, b, other, A);
-    gsApply<L>(s1, B, xs, part, zero, useOther, omega);
-    s0 = s2;
-    s1 = s3;
-  }
-  if (k < ns) gsApply<L>(s0, A, xs, part, zero, useOther, omega);
-}
 
 }  // namespace dev
 }  // namespace nodals

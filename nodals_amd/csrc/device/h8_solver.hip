@@ -184,7 +184,7 @@ H8Options parseH8Args(int argc, const char* const* argv) {
     else if (a == "--amg-mcgs-fine-sweeps") o.amgMcgsFineSweeps = inum(next());
     else if (a == "--amg-mcgs-coarse-sweeps") o.amgMcgsCoarseSweeps = inum(next());
     else if (a == "--amg-mcgs-order") o.amgMcgsOrder = next();
-    else if (a == "--amg-mcgs-fuse-nnz") o.amgMcgsFuseNnz = (long long)num(next());
+    else if (a == "--amg-mcgs-fuse-nnz") (void)next();  // accepted; small levels are one dense product
     else if (a == "--momentum-work") o.momentumWork = next();
     else if (a == "--mom-sweeps") o.momSweeps = inum(next());
     else if (a == "--run-mode") o.runMode = next();
@@ -667,7 +667,6 @@ void H8Solver::setupAmg() {
   so.mcgsFineSweeps = opt_.amgMcgsFineSweeps;
   so.mcgsCoarseSweeps = opt_.amgMcgsCoarseSweeps;
   so.mcgsOrder = opt_.amgMcgsOrder;
-  so.mcgsFuseNnz = opt_.amgMcgsFuseNnz;
   Coloring fineColor;
   if (so.kind == "mcgs") fineColor = greedyColoring32(nc_, F_.row.data(), F_.col.data());
   const Coloring* fc = so.kind == "mcgs" ? &fineColor : nullptr;
@@ -677,39 +676,36 @@ void H8Solver::setupAmg() {
     FineView<double, double> v;
     v.n = nc_;
     v.lanes = fineLanes_;
-    v.meanRow = fineMeanRow_;
     v.row = frow_.data();
     v.col = fcol_.data();
     v.val = fval_.data();
     v.diag = fdiag_.data();
     v.l1 = fl1_.data();
-    amg64_->setFine(v);
+    amg64_->setFine(v, F_.row.data(), F_.col.data(), fc);
   } else if (opt_.amgPrecision == "fp32") {
     amg32_ = std::make_unique<DevAmg<float, float>>();
     amg32_->setup(H_, nc_, so, fc);
     FineView<float, float> v;
     v.n = nc_;
     v.lanes = fineLanes_;
-    v.meanRow = fineMeanRow_;
     v.row = frow_.data();
     v.col = fcol_.data();
     v.val = fvalf_.data();
     v.diag = fdiagf_.data();
     v.l1 = fl1f_.data();
-    amg32_->setFine(v);
+    amg32_->setFine(v, F_.row.data(), F_.col.data(), fc);
   } else {
     amgb_ = std::make_unique<DevAmg<bf16, float>>();
     amgb_->setup(H_, nc_, so, fc);
     FineView<bf16, float> v;
     v.n = nc_;
     v.lanes = fineLanes_;
-    v.meanRow = fineMeanRow_;
     v.row = frow_.data();
     v.col = fcol_.data();
     v.val = fvalb_.data();
     v.diag = fdiagf_.data();
     v.l1 = fl1f_.data();
-    amgb_->setFine(v);
+    amgb_->setFine(v, F_.row.data(), F_.col.data(), fc);
   }
 }
 
@@ -929,6 +925,11 @@ void H8Solver::refreshOn(hipStream_t s) {
 #undef NODALS_REFRESH_P
 #undef NODALS_REFRESH
   NODALS_LAUNCHED();
+  if (opt_.amgSmoother == "mcgs") {  // the smoother's slots mirror the values
+    if (amg64_) amg64_->fineChanged(s);
+    if (amg32_) amg32_->fineChanged(s);
+    if (amgb_) amgb_->fineChanged(s);
+  }
 }
 
 void H8Solver::fineApply(hipStream_t s, const double* x, double* y) {

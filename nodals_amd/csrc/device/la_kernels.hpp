@@ -22,6 +22,56 @@ __device__ __forceinline__ T groupSum(T v, int lanes) {
   return v;
 }
 
+// Sum over groups of L consecutive lanes (every lane gets it) with cross-lane
+// moves inside the registers: quad swaps, half-row and row mirrors (the
+// mirrored lanes hold equal partial sums already), then 16- and 32-lane swaps.
+template <int CTRL>
+__device__ __forceinline__ int dppMove(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dppMove(float v) {
+  return __int_as_float(dppMove<CTRL>(__float_as_int(v)));
+}
+__device__ __forceinline__ double fromWords(unsigned lo, unsigned hi) {
+  return __longlong_as_double(((long long)(int)hi << 32) | lo);
+}
+template <int CTRL>
+__device__ __forceinline__ double dppMove(double v) {
+  const long long b = __double_as_longlong(v);
+  return fromWords((unsigned)dppMove<CTRL>((int)b), (unsigned)dppMove<CTRL>((int)(b >> 32)));
+}
+__device__ __forceinline__ float swapAdd16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double swapAdd16(double v) {
+  const long long b = __double_as_longlong(v);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
+}
+__device__ __forceinline__ float swapAdd32(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double swapAdd32(double v) {
+  const long long b = __double_as_longlong(v);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
+}
+template <int L, class T>
+__device__ __forceinline__ T laneSum(T v) {
+  if constexpr (L >= 2) v += dppMove<0xB1>(v);   // quad_perm [1,0,3,2]
+  if constexpr (L >= 4) v += dppMove<0x4E>(v);   // quad_perm [2,3,0,1]
+  if constexpr (L >= 8) v += dppMove<0x141>(v);  // row_half_mirror
+  if constexpr (L >= 16) v += dppMove<0x140>(v);  // row_mirror
+  if constexpr (L >= 32) v = swapAdd16(v);
+  if constexpr (L >= 64) v = swapAdd32(v);
+  return v;
+}
+
 // A lane's share of a CSR row product: s = sum of val(k) * gather(col[k])
 // over k = k0, k0 + LANES, ... < e, accumulated in exactly that order (the
 // order of the one-at-a-time loop, so results are bit-identical to it).  Each
@@ -343,97 +393,6 @@ __global__ void __launch_bounds__(256) k_row_l1(int n, const int* __restrict__ r
   if (lane == 0) l1[r] = s;
 }
 
-// One multicolour Gauss-Seidel colour: rows crow[begin..begin+count), or
-// rows begin..begin+count when crow is null (operator numbered in colour
-// order).
-// x_i <- x_i + omega ((b_i - sum_{j!=i} a_ij x_j)/d_i - x_i)
-template <int LANES, class TM, class TV>
-__global__ void __launch_bounds__(256) k_mcgs_color(int begin, int count, const int* __restrict__ crow,
-                                                    const int* __restrict__ row, const int* __restrict__ col,
-                                                    const TM* __restrict__ val, const TV* __restrict__ diag,
-                                                    const TV* __restrict__ b, TV* __restrict__ x, double omega) {
-  const int gid = blockIdx.x * 256 + threadIdx.x;
-  const int q = gid / LANES;
-  const int lane = gid % LANES;
-  if (q >= count) return;
-  const int i = crow ? crow[begin + q] : begin + q;  // no list: the colour is a contiguous row range
-  // the row's own b, diagonal and value do not depend on the row product:
-  // their loads are issued with the row's, not after the reduction
-  const TV bi = b[i], di = diag[i], old = x[i];
-  TV s = rowDot<LANES, TV>(
-      row[i] + lane, row[i + 1], col, i, [&](int k) { return ld<TV>(val, k); }, [&](int j) { return x[j]; });
-  s = groupSum(s, LANES);
-  if (lane == 0) {
-    const TV gs = (bi - s) / di;
-    x[i] = old + (TV)omega * (gs - old);
-  }
-}
-
-// A whole MCGS smoothing call of one small level in one workgroup, from x =
-// 0: `sweeps` sweeps of forward (order 0), backward (1) or forward then
-// backward (2) colour passes over the level numbered in colour order (colour
-// c is rows [coff[c], coff[c+1])), with a barrier between colours instead of
-// a launch per colour.  The iterate, the row pointers, the right-hand side
-// and the diagonal are staged in LDS, so a row's chain is one global load
-// (its columns and values) between LDS reads.  Colour c's rows use
-// clanes[c] lanes each, the lanes of k_mcgs_color's launch for that colour,
-// and the same rowDot/groupSum, so the result is bit-identical to the
-// launch-per-colour passes.  Dynamic LDS: n (3 sizeof(TV) + 4) + 4 bytes.
-template <int L, class TM, class TV>
-__device__ __forceinline__ void mcgsRowsLds(int begin, int count, const int* rs, const int* __restrict__ col,
-                                            const TM* __restrict__ val, const TV* ds, const TV* bs, TV* xs,
-                                            double omega) {
-  const int lane = threadIdx.x % L;
-  for (int q = threadIdx.x / L; q < count; q += blockDim.x / L) {
-    const int i = begin + q;
-    const TV bi = bs[i], di = ds[i], old = xs[i];
-    TV s = rowDot<L, TV>(
-        rs[i] + lane, rs[i + 1], col, i, [&](int k) { return ld<TV>(val, k); }, [&](int j) { return xs[j]; });
-    s = groupSum(s, L);
-    if (lane == 0) {
-      const TV gs = (bi - s) / di;
-      xs[i] = old + (TV)omega * (gs - old);
-    }
-  }
-}
-
-template <class TM, class TV>
-__global__ void __launch_bounds__(1024) k_mcgs_level_wg(int n, const int* __restrict__ row, const int* __restrict__ col,
-                                                        const TM* __restrict__ val, const TV* __restrict__ diag,
-                                                        const TV* __restrict__ b, TV* __restrict__ x, int ncolors,
-                                                        const int* __restrict__ coff, const int* __restrict__ clanes,
-                                                        int sweeps, int order, double omega) {
-  extern __shared__ unsigned char ldsRaw[];
-  TV* xs = reinterpret_cast<TV*>(ldsRaw);
-  TV* bs = xs + n;
-  TV* ds = bs + n;
-  int* rs = reinterpret_cast<int*>(ds + n);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    xs[i] = TV(0);
-    bs[i] = b[i];
-    ds[i] = diag[i];
-  }
-  for (int i = threadIdx.x; i <= n; i += blockDim.x) rs[i] = row[i];
-  __syncthreads();
-  for (int sw = 0; sw < sweeps; ++sw)
-    for (int pass = 0; pass < 2; ++pass) {
-      if ((pass == 0 && order == 1) || (pass == 1 && order == 0)) continue;
-      for (int q = 0; q < ncolors; ++q) {
-        const int c = pass == 1 ? ncolors - 1 - q : q;
-        const int begin = coff[c], count = coff[c + 1] - begin;
-        switch (clanes[c]) {
-          case 4: mcgsRowsLds<4, TM, TV>(begin, count, rs, col, val, ds, bs, xs, omega); break;
-          case 8: mcgsRowsLds<8, TM, TV>(begin, count, rs, col, val, ds, bs, xs, omega); break;
-          case 16: mcgsRowsLds<16, TM, TV>(begin, count, rs, col, val, ds, bs, xs, omega); break;
-          case 32: mcgsRowsLds<32, TM, TV>(begin, count, rs, col, val, ds, bs, xs, omega); break;
-          default: mcgsRowsLds<64, TM, TV>(begin, count, rs, col, val, ds, bs, xs, omega); break;
-        }
-        __syncthreads();
-      }
-    }
-  for (int i = threadIdx.x; i < n; i += blockDim.x) x[i] = xs[i];
-}
-
 template <class T>
 __global__ void k_diag_gather(int n, const int* __restrict__ diagPos, const T* __restrict__ val, T* __restrict__ d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -567,21 +526,6 @@ void rowL1(hipStream_t s, int lanes, int n, const int* row, const TM* val, TV* l
     case 16: hipLaunchKernelGGL((k_row_l1<16, TM, TV>), grid, 256, 0, s, n, row, val, l1); break;
     case 32: hipLaunchKernelGGL((k_row_l1<32, TM, TV>), grid, 256, 0, s, n, row, val, l1); break;
     default: hipLaunchKernelGGL((k_row_l1<64, TM, TV>), grid, 256, 0, s, n, row, val, l1); break;
-  }
-  NODALS_LAUNCHED();
-}
-
-template <class TM, class TV>
-void mcgsColor(hipStream_t s, int lanes, int begin, int count, const int* crow, const int* row, const int* col,
-               const TM* val, const TV* diag, const TV* b, TV* x, double omega) {
-  if (count <= 0) return;
-  const int grid = blocksFor((long long)count * lanes);
-  switch (lanes) {
-    case 4: hipLaunchKernelGGL((k_mcgs_color<4, TM, TV>), grid, 256, 0, s, begin, count, crow, row, col, val, diag, b, x, omega); break;
-    case 8: hipLaunchKernelGGL((k_mcgs_color<8, TM, TV>), grid, 256, 0, s, begin, count, crow, row, col, val, diag, b, x, omega); break;
-    case 16: hipLaunchKernelGGL((k_mcgs_color<16, TM, TV>), grid, 256, 0, s, begin, count, crow, row, col, val, diag, b, x, omega); break;
-    case 32: hipLaunchKernelGGL((k_mcgs_color<32, TM, TV>), grid, 256, 0, s, begin, count, crow, row, col, val, diag, b, x, omega); break;
-    default: hipLaunchKernelGGL((k_mcgs_color<64, TM, TV>), grid, 256, 0, s, begin, count, crow, row, col, val, diag, b, x, omega); break;
   }
   NODALS_LAUNCHED();
 }

@@ -110,13 +110,13 @@ SysSolver::SysSolver(int n, const std::int64_t* row, const std::int32_t* col, co
     FineView<double, double> v;
     v.n = n;
     v.lanes = lanes_;
-    v.meanRow = meanRow_;
     v.row = row_.data();
     v.col = col_.data();
     v.val = val_.data();
     v.diag = diag_.data();
     v.l1 = l1_.data();
-    amg64_->setFine(v);
+    amg64_->setFine(v, r32.data(), A_.col.data(), pfc);
+      amg64_->fineChanged(stream_);
   } else {
     std::vector<float> df(A_.diag.begin(), A_.diag.end()), lf(l1.begin(), l1.end());
     diagf_.upload(df);
@@ -131,14 +131,13 @@ SysSolver::SysSolver(int n, const std::int64_t* row, const std::int32_t* col, co
       FineView<float, float> v;
       v.n = n;
       v.lanes = lanes_;
-      v.meanRow = meanRow_;
-    v.meanRow = meanRow_;
       v.row = row_.data();
       v.col = col_.data();
       v.val = valf_.data();
       v.diag = diagf_.data();
       v.l1 = l1f_.data();
-      amg32_->setFine(v);
+      amg32_->setFine(v, r32.data(), A_.col.data(), pfc);
+      amg32_->fineChanged(stream_);
     } else {
       std::vector<bf16> vb(nnz);
       for (std::size_t k = 0; k < nnz; ++k) vb[k] = floatToBf16((float)A_.val[k]);
@@ -148,14 +147,13 @@ SysSolver::SysSolver(int n, const std::int64_t* row, const std::int32_t* col, co
       FineView<bf16, float> v;
       v.n = n;
       v.lanes = lanes_;
-      v.meanRow = meanRow_;
-    v.meanRow = meanRow_;
       v.row = row_.data();
       v.col = col_.data();
       v.val = valb_.data();
       v.diag = diagf_.data();
       v.l1 = l1f_.data();
-      amgb_->setFine(v);
+      amgb_->setFine(v, r32.data(), A_.col.data(), pfc);
+      amgb_->fineChanged(stream_);
     }
   }
   NODALS_HIP(hipStreamSynchronize(stream_));

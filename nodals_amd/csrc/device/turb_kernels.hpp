@@ -8,7 +8,7 @@
 // k_turb_wall_trace), then one
 // gather per vertex row that sums its entries over the blocks, forms the
 // row-L1 relaxation and writes the sweep operator, diagonal and right-hand
-// side (k_turb_gather); the coloured sweeps are k_mcgs_color; k_turb_floor
+// side (k_turb_gather); the coloured sweeps are k_gs_colour; k_turb_floor
 // applies the floor.  No atomics in the assembly: every entry is summed by
 // exactly one lane in a fixed order.
 //

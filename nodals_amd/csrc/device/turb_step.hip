@@ -179,7 +179,12 @@ void H8Solver::turbInit(const TurbParams& P) {
   st->blk.alloc(nb * 64);
   st->brhs.alloc(nb * 8);
   st->val.alloc(T.col.size());
-  if (P.sweepFp32) st->valF.alloc(T.col.size());
+  {
+    const GsLayout G = gsLayout(T.coloring.ncolors, T.coloring.offset, T.coloring.rows.data(), T.coloring.color,
+                                T.row.data(), T.col.data(), GsHalf::all);
+    if (P.sweepFp32) st->gsF.upload(G, nullptr);
+    else st->gs.upload(G, nullptr);
+  }
   st->diag.alloc((std::size_t)T.nvert);
   st->rhs.alloc((std::size_t)T.nvert);
   std::vector<double> k0((std::size_t)T.nS, 0.0), w0((std::size_t)T.nS, 0.0);
@@ -265,20 +270,21 @@ int H8Solver::turbEquation(int eq, double* rel0, double* rel1) {
   if (rel0) *rel0 = relResid();
   // the fixed sweeps (sweeps x colours launches on fixed buffers) replay
   // from one captured graph per equation
-  const double meanRow = (double)T.col.size() / std::max(T.nvert, 1);
   const int sweeps = eq == 0 ? P.kSweeps : P.omegaSweeps;
-  if (P.sweepFp32) cast<float, double>(s, (long long)T.col.size(), st.val.data(), st.valF.data());
+  if (P.sweepFp32) st.gsF.fill(s, st.val.data());
+  else st.gs.fill(s, st.val.data());
   st.sweepGraph[eq].run(s, graphKey({x, st.val.data(), st.rhs.data()}, sweeps * 4.0 + P.gsOmega), [&]() {
-    for (int sw = 0; sw < sweeps; ++sw)
-      for (int c = 0; c < T.coloring.ncolors; ++c) {
-        const int b = st.colorOff[(std::size_t)c], n = st.colorOff[(std::size_t)c + 1] - b;
-        if (P.sweepFp32)
-          mcgsColor<float, double>(s, lanesFor(meanRow, n), b, n, st.crows.data(), st.row.data(), st.col.data(),
-                                   st.valF.data(), st.diag.data(), st.rhs.data(), x, P.gsOmega);
-        else
-          mcgsColor<double, double>(s, lanesFor(meanRow, n), b, n, st.crows.data(), st.row.data(),
-                                    st.col.data(), st.val.data(), st.diag.data(), st.rhs.data(), x, P.gsOmega);
-      }
+    auto sweep = [&](const auto& G) {
+      for (int sw = 0; sw < sweeps; ++sw)
+        for (int c = 0; c < T.coloring.ncolors; ++c) {
+          const int b = st.colorOff[(std::size_t)c], n = st.colorOff[(std::size_t)c + 1] - b;
+          gsColour(s, G.colour[(std::size_t)c], b, n, (const int*)st.crows.data(), G.col.data(), G.val.data(),
+                   (const double*)st.diag.data(), (const double*)st.rhs.data(), x, (const double*)nullptr,
+                   (double*)nullptr, false, P.gsOmega);
+        }
+    };
+    if (P.sweepFp32) sweep(st.gsF);
+    else sweep(st.gs);
   });
   if (rel1) *rel1 = relResid();
   hipLaunchKernelGGL(k_turb_floor, blocksFor(T.nvert), 256, 0, s, T.nvert, eq == 0 ? P.kFloor : P.omegaFloor, x,

@@ -15,6 +15,7 @@
 
 #include "../host/turb_setup.hpp"
 #include "common.hpp"
+#include "gs_ell.hpp"
 
 namespace nodals {
 
@@ -47,7 +48,9 @@ struct TurbState {
   // (the reference holds one count for both, SST24B_ACTIVE_POINTS)
   int omegaFitPoints = 5;
   DBuf<double> vdist;  // vertex wall distances (duct mode), empty for the straight pipe
-  DBuf<float> valF;    // FP32 copy of val for --sst-sweep-precision fp32
+  // the sweeps' slots of val, in FP64 or (--sst-sweep-precision fp32) FP32
+  dev::GsSlots<double> gs;
+  dev::GsSlots<float> gsF;
   DBuf<double> resid;  // residual of a scalar_solve norm
   const double* vdistPtr() const { return vdist.size() ? vdist.data() : nullptr; }
   std::vector<int> colorOff;
