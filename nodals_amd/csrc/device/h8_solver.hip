@@ -1143,16 +1143,19 @@ void H8Solver::ransBlocks() {
   A.ufix = fixedVal_.data();
   A.radius = S_.pipe.R;
   A.nu = S_.pipe.nu;
-  A.mixing = opt_.mixingLength ? 1 : 0;
   A.mixScale = opt_.mixlenScale;
-  A.supg = opt_.supg ? 1 : 0;
   A.tauScale = opt_.supgTauScale;
   A.magic = opt_.supgMagic;
   A.cbuf = cbuf_.data();
   A.stats = ransStats_.data();
-  // one wavefront per cell, eight per CU resident across the chip
-  const int grid = std::max(1, std::min(nc_, 8 * std::max(cuCount_, 1)));
-  hipLaunchKernelGGL(dev::k_rans64, grid, 64, 0, stream_, A, dev::collapsed64());
+  // one wavefront per cell, two blocks of four resident on each CU
+  const int grid = std::max(1, std::min((nc_ + 3) / 4, 2 * std::max(cuCount_, 1)));
+  if (opt_.mixingLength && opt_.supg)
+    hipLaunchKernelGGL((dev::k_rans64<true, true>), grid, 256, 0, stream_, A, dev::collapsed64());
+  else if (opt_.mixingLength)
+    hipLaunchKernelGGL((dev::k_rans64<true, false>), grid, 256, 0, stream_, A, dev::collapsed64());
+  else
+    hipLaunchKernelGGL((dev::k_rans64<false, true>), grid, 256, 0, stream_, A, dev::collapsed64());
   NODALS_LAUNCHED();
 }
 

@@ -72,6 +72,60 @@ __device__ __forceinline__ T laneSum(T v) {
   return v;
 }
 
+// Maximum over the wavefront.
+__device__ __forceinline__ double waveMax(double v) {
+  v = fmax(v, dppMove<0xB1>(v));
+  v = fmax(v, dppMove<0x4E>(v));
+  v = fmax(v, dppMove<0x141>(v));
+  v = fmax(v, dppMove<0x140>(v));
+  for (int o = 16; o < 64; o <<= 1) v = fmax(v, __shfl_xor(v, o));
+  return v;
+}
+
+// Transposing reduction: every lane of a group of L holds N partial sums
+// v[0..N); afterwards lane l of the group holds the group's totals of entries
+// (N / L) l .. (N / L) l + N / L - 1 in v[0..N / L).  Each stage halves the
+// entries: a lane keeps the half its bit selects and adds its partner's
+// partial sums of it, N - 1 exchanges in all instead of N log2 L.  Partners
+// are the mirrored lanes, which differ in the stage's bit (and in lower ones,
+// whose lanes still hold the same entries); at 16 and 32 lanes one swap of
+// rows or halves serves both partners.
+__device__ __forceinline__ double swapPair16(double a, double b) {
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
+}
+__device__ __forceinline__ double swapPair32(double a, double b) {
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double mirrorPair(double a, double b, bool upper) {
+  return (upper ? b : a) + dppMove<CTRL>(upper ? a : b);
+}
+template <int N, int L>
+__device__ __forceinline__ void laneReduceScatter(double (&v)[N], int lane) {
+  static_assert(N >= L && (L == 32 || L == 64), "entries over 32 or 64 lanes");
+  if (L == 64) {
+#pragma unroll
+    for (int p = 0; p < N / 2; ++p) v[p] = swapPair32(v[p], v[p + N / 2]);
+  }
+  constexpr int n4 = L == 64 ? N / 2 : N;  // entries at the 16-lane stage
+#pragma unroll
+  for (int p = 0; p < n4 / 2; ++p) v[p] = swapPair16(v[p], v[p + n4 / 2]);
+#pragma unroll
+  for (int p = 0; p < n4 / 4; ++p) v[p] = mirrorPair<0x140>(v[p], v[p + n4 / 4], lane & 8);
+#pragma unroll
+  for (int p = 0; p < n4 / 8; ++p) v[p] = mirrorPair<0x141>(v[p], v[p + n4 / 8], lane & 4);
+#pragma unroll
+  for (int p = 0; p < n4 / 16; ++p) v[p] = mirrorPair<0x1B>(v[p], v[p + n4 / 16], lane & 2);
+#pragma unroll
+  for (int p = 0; p < n4 / 32; ++p) v[p] = mirrorPair<0xB1>(v[p], v[p + n4 / 32], lane & 1);
+}
+
 // A lane's share of a CSR row product: s = sum of val(k) * gather(col[k])
 // over k = k0, k0 + LANES, ... < e, accumulated in exactly that order (the
 // order of the one-at-a-time loop, so results are bit-identical to it).  Each
