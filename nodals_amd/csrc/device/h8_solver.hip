@@ -1130,6 +1130,37 @@ void H8Solver::sstGeometry() {
   sstQuad_.upload(keast24());
 }
 
+dev::SstVolArgs H8Solver::sstVolArgs(int equation, double kFloor, double omegaFloor, int deviatoric) {
+  dev::SstVolArgs A{};
+  A.nc = nc_;
+  A.cref = cref_.data();
+  A.cinvJ = cinvJ_.data();
+  A.cdet = cdet_.data();
+  A.cxy = sstXY_.data();
+  A.u = u_.data();
+  A.ufix = fixedVal_.data();
+  A.quad = sstQuad_.data();
+  A.radius = S_.pipe.R;
+  A.nu = S_.pipe.nu;
+  A.equation = equation;
+  A.kFloor = kFloor;
+  A.omFloor = omegaFloor;
+  A.deviatoric = deviatoric;
+  return A;
+}
+
+// The same with the k-omega step's own fields (one scalar per mesh entity).
+dev::SstVolArgs H8Solver::turbVolArgs(int equation) {
+  TurbState& st = *turb_;
+  const TurbParams& P = st.P;
+  dev::SstVolArgs A = sstVolArgs(equation, P.kFloor, P.omegaFloor, P.deviatoric ? 1 : 0);
+  A.kf = A.kfix = st.k.data();
+  A.wf = A.wfix = st.w.data();
+  A.sref = st.sref.data();
+  A.vdist = st.vdistPtr();
+  return A;
+}
+
 void H8Solver::ransBlocks() {
   if (opt_.mixingLength) sstGeometry();
   dev::RansArgs A;
@@ -1224,11 +1255,14 @@ void H8Solver::sstVolume(int equation, const std::vector<double>& kFree, const s
   dwf.upload(wf);
   dmat.alloc((std::size_t)nc_ * 64);
   drhs.alloc((std::size_t)nc_ * 8);
-  hipLaunchKernelGGL(k_sst_volume, (nc_ + 3) / 4, 256, 0, stream_, nc_, cref_.data(), cinvJ_.data(), cdet_.data(),
-                     sstXY_.data(), u_.data(), fixedVal_.data(), dk.data(), dkf.data(), dw.data(), dwf.data(),
-                     sstQuad_.data(), S_.pipe.R, S_.pipe.nu, equation, kFloor, omegaFloor, deviatoric, dmat.data(),
-                     drhs.data());
-  NODALS_LAUNCHED();
+  SstVolArgs A = sstVolArgs(equation, kFloor, omegaFloor, deviatoric);
+  A.kf = dk.data();
+  A.kfix = dkf.data();
+  A.wf = dw.data();
+  A.wfix = dwf.data();
+  A.mat = dmat.data();
+  A.rhs = drhs.data();
+  dev::launchSstVolume(stream_, A);
   sync();
   mat = dmat.host();
   rhs = drhs.host();

@@ -22,6 +22,7 @@
 #include "amg.hpp"
 #include "gnn.hpp"
 #include "krylov.hpp"
+#include "sst_volume.hpp"
 #include "turb_step.hpp"
 
 namespace nodals {
@@ -337,6 +338,8 @@ class H8Solver {
   // statistics [nc][4].
   DBuf<double> ch2_, ransStats_;
   void ransBlocks();
+  dev::SstVolArgs sstVolArgs(int equation, double kFloor, double omegaFloor, int deviatoric);
+  dev::SstVolArgs turbVolArgs(int equation);
   // DG weak inlet (--dg-inlet): inlet faces, their right-hand sides and the
   // rows those reach
   DBuf<int> dgCell_, dgLf_, dgRows_, dgOff_, dgList_;

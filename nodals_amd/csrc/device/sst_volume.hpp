@@ -8,9 +8,7 @@
 // (reference kernel sst_tet_volume,
 // turbulence/sst_gpu_v2/source/puretet_profile5_eq5_hxt5b/modules/transport/
 // tet_volume_kernel.inc:1-30, with volume_coefficients,
-// modules/transport/portable/transport_core.hpp:14-25).  One wavefront per
-// cell: lanes 0..23 evaluate the points, then lane 8a+b forms A_ab and
-// lanes 0..7 b_a from the per-point terms staged in LDS; every cell writes
+// modules/transport/portable/transport_core.hpp:14-25).  Every cell writes
 // its own 8x8 block (no atomics).
 #pragma once
 
@@ -20,6 +18,7 @@
 #include <array>
 #include <vector>
 
+#include "la_kernels.hpp"
 #include "sst_physics.hpp"
 
 namespace nodals {
@@ -95,45 +94,77 @@ __device__ inline void p1bf3Basis(const double l[4], double phi[8], double gr[8]
 // (modules/coupling/implicit_dev_volume_tet.inc:1-68):
 //   dmat[c][ab][3i+j] = sum_q w_q det (nu + nu_t)
 //                       (d_j phi_a d_i phi_b - (2/3) d_i phi_a d_j phi_b).
-static __global__ void __launch_bounds__(256) k_sst_volume(
-    int nc, const int* __restrict__ cref, const double* __restrict__ cinvJ, const double* __restrict__ cdet,
-    const double* __restrict__ cxy, const double* __restrict__ u, const double* __restrict__ ufix,
-    const double* __restrict__ kf, const double* __restrict__ kfix, const double* __restrict__ wf,
-    const double* __restrict__ wfix, const double* __restrict__ quad, double radius, double nu, int equation,
-    double kFloor, double omFloor, int deviatoric, double* mat, double* __restrict__ rhs,
-    const int* __restrict__ sref = nullptr, double nuBase = 0.0, const double* conv = nullptr,
-    const double* __restrict__ vdist = nullptr, double* __restrict__ dmat = nullptr) {
-  __shared__ double PH[4][kSstQ][8], GP[4][kSstQ][8][3], DW[4][kSstQ], RW[4][kSstQ], SW[4][kSstQ], NW[4][kSstQ];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c = blockIdx.x * 4 + wv;
-  const bool live = c < nc;
-  if (live && lane < kSstQ) {
-    const int q = lane;
-    const double* Q = quad + 5 * q;
-    const double l[4] = {Q[0], Q[1], Q[2], Q[3]};
-    double phi[8], gr[8][3];
+//
+// Two cells per wavefront, 32 lanes a cell, one lane a quadrature point (the
+// last eight idle with zero weights).  A lane evaluates its point, forms all 64
+// products of the block from registers, and a transposing reduction over the
+// 32 lanes leaves entries 2l and 2l + 1 in lane l, so the block is written
+// in one coalesced store and no LDS is needed.  The point evaluation (the SST
+// state, two tanh and a dozen divisions) is then the time.  The form with
+// 24 of 64 lanes evaluating and 64 lanes each looping over points staged in
+// LDS took 334 us on the 40k pipe; this one 104 us.
+//
+// The deviatoric tensor is the 24 x 24 product G^T N G of the points'
+// gradients (row 3a + i): DMAT stages G and N in LDS and forms it with
+// v_mfma_f64_16x16x4 (four tiles, six steps; operand lane l supplies row l%16
+// of k = l/16, accumulator register r holds row l/16 + 4r, column l%16), then
+// combines entries (3a+j, 3b+i) and (3a+i, 3b+j) from LDS.  On the 207k helix
+// an iteration's three calls (one with the tensor) took 6.6 ms, now 1.9 ms.
+struct SstVolArgs {
+  int nc;
+  const int* cref;
+  const double *cinvJ, *cdet, *cxy, *u, *ufix, *kf, *kfix, *wf, *wfix, *quad;
+  double radius, nu;
+  int equation;
+  double kFloor, omFloor;
+  int deviatoric;
+  double *mat, *rhs;
+  const int* sref;
+  double nuBase;
+  const double *conv, *vdist;
+  double* dmat;
+};
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <bool DMAT>
+static __global__ void __launch_bounds__(256, 2) k_sst_volume(SstVolArgs A) {
+  constexpr int kComp = 24, kPad = 25;  // a point's gradient components, padded rows
+  __shared__ double GS[DMAT ? 8 * kSstQ * kPad : 1], NS[DMAT ? 8 * kSstQ : 1];
+  const int lane = threadIdx.x & 63, half = lane >> 5, lq = lane & 31;
+  const int wave = threadIdx.x >> 6, slot = 2 * wave + half;
+  const int cell = blockIdx.x * 8 + slot;
+  const bool live = cell < A.nc;
+  const int c = live ? cell : A.nc - 1;
+  const bool point = live && lq < kSstQ;
+  const double* Q = A.quad + 5 * (lq < kSstQ ? lq : 0);
+  const double l[4] = {Q[0], Q[1], Q[2], Q[3]};
+  double phi[8], G[8][3];
+  double DWq, RWq, SWq, NWq;
+  {
+    double gr[8][3];
     p1bf3Basis(l, phi, gr);
-    const double* I = cinvJ + (long long)c * 9;
+    const double* I = A.cinvJ + (long long)c * 9;
     double gu[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, gk[3] = {0, 0, 0}, gw[3] = {0, 0, 0}, kv = 0, wvv = 0;
+#pragma unroll
     for (int a = 0; a < 8; ++a) {
-      const int r = cref[(long long)c * 8 + a];
-      const double* U = r >= 0 ? u + 3ll * r : ufix + 3ll * (-r - 1);
+      const int r = A.cref[(long long)c * 8 + a];
+      const double* U = r >= 0 ? A.u + 3ll * r : A.ufix + 3ll * (-r - 1);
       double Ka, Wa;
-      if (sref) {
-        const int g = sref[(long long)c * 8 + a];
-        Ka = kf[g];
-        Wa = wf[g];
+      if (A.sref) {
+        const int g = A.sref[(long long)c * 8 + a];
+        Ka = A.kf[g];
+        Wa = A.wf[g];
       } else {
-        Ka = r >= 0 ? kf[r] : kfix[-r - 1];
-        Wa = r >= 0 ? wf[r] : wfix[-r - 1];
+        Ka = r >= 0 ? A.kf[r] : A.kfix[-r - 1];
+        Wa = r >= 0 ? A.wf[r] : A.wfix[-r - 1];
       }
       const double pa = phi[a];
-      PH[wv][q][a] = pa;
       kv += Ka * pa;
       wvv += Wa * pa;
       for (int d = 0; d < 3; ++d) {
         const double gd = gr[a][0] * I[d] + gr[a][1] * I[3 + d] + gr[a][2] * I[6 + d];
-        GP[wv][q][a][d] = gd;
+        G[a][d] = gd;
         gk[d] += Ka * gd;
         gw[d] += Wa * gd;
         gu[d] += U[0] * gd;
@@ -142,59 +173,129 @@ static __global__ void __launch_bounds__(256) k_sst_volume(
       }
     }
     double dq;
-    if (vdist) {  // P1 interpolation of the vertex wall-distance field
+    if (A.vdist) {  // P1 interpolation of the vertex wall-distance field
       double dd = 0;
-      for (int a = 0; a < 4; ++a) dd += l[a] * vdist[sref[(long long)c * 8 + a]];
-      dq = sst::floorDistance(fmax(0.0, dd), radius);
+      for (int a = 0; a < 4; ++a) dd += l[a] * A.vdist[A.sref[(long long)c * 8 + a]];
+      dq = sst::floorDistance(fmax(0.0, dd), A.radius);
     } else {
       double xq = 0, yq = 0;
       for (int a = 0; a < 4; ++a) {
-        xq += l[a] * cxy[(long long)c * 8 + 2 * a];
-        yq += l[a] * cxy[(long long)c * 8 + 2 * a + 1];
+        xq += l[a] * A.cxy[(long long)c * 8 + 2 * a];
+        yq += l[a] * A.cxy[(long long)c * 8 + 2 * a + 1];
       }
-      dq = sst::pipeDistance(xq, yq, radius);
+      dq = sst::pipeDistance(xq, yq, A.radius);
     }
-    const sst::Local s = sst::local(dq, nu, gu, kv, wvv, gk, gw, kFloor, omFloor, deviatoric != 0);
-    const double wt = cdet[c] * Q[4];
-    const bool isK = equation == 0;
-    if (equation == 2) {
-      DW[wv][q] = wt * s.nut;
-      RW[wv][q] = 0.0;
-      SW[wv][q] = 0.0;
-      NW[wv][q] = (nu + s.nut) * wt;
+    const sst::Local s = sst::local(dq, A.nu, gu, kv, wvv, gk, gw, A.kFloor, A.omFloor, A.deviatoric != 0);
+    const double wt = A.cdet[c] * Q[4];
+    const bool isK = A.equation == 0;
+    if (A.equation == 2) {
+      DWq = wt * s.nut;
+      RWq = 0.0;
+      SWq = 0.0;
+      NWq = (A.nu + s.nut) * wt;
     } else {
-      DW[wv][q] = wt * ((isK ? s.sigmaK : s.sigmaW) * s.nut + nuBase);
-      RW[wv][q] = wt * (isK ? s.reactK : s.reactOmega);
-      SW[wv][q] = wt * (isK ? s.pk : s.srcOmega);
+      DWq = wt * ((isK ? s.sigmaK : s.sigmaW) * s.nut + A.nuBase);
+      RWq = wt * (isK ? s.reactK : s.reactOmega);
+      SWq = wt * (isK ? s.pk : s.srcOmega);
+      NWq = 0.0;
+    }
+    if (!point) DWq = RWq = SWq = NWq = 0.0;
+  }
+  if (DMAT) {
+    if (lq < kSstQ) {
+      double* g = GS + ((long long)slot * kSstQ + lq) * kPad;
+      for (int a = 0; a < 8; ++a)
+        for (int d = 0; d < 3; ++d) g[3 * a + d] = G[a][d];
+      NS[slot * kSstQ + lq] = NWq;
     }
   }
-  __syncthreads();
-  if (!live) return;
   {
+    double v[64];
+#pragma unroll
+    for (int a = 0; a < 8; ++a) {
+      const double h0 = DWq * G[a][0], h1 = DWq * G[a][1], h2 = DWq * G[a][2], hp = RWq * phi[a];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) v[8 * a + b] = h0 * G[b][0] + h1 * G[b][1] + h2 * G[b][2] + hp * phi[b];
+    }
+    laneReduceScatter<64, 32>(v, lane);
+    if (live) {
+      const long long o = (long long)c * 64 + 2 * lq;
+      A.mat[o] = A.conv ? v[0] + A.conv[o] : v[0];
+      A.mat[o + 1] = A.conv ? v[1] + A.conv[o + 1] : v[1];
+    }
+  }
+  if (A.rhs) {
+    double r[8];
+#pragma unroll
+    for (int a = 0; a < 8; ++a) r[a] = SWq * phi[a];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) r[p] = mirrorPair<0x140>(r[p], r[p + 4], lane & 8);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) r[p] = mirrorPair<0x141>(r[p], r[p + 2], lane & 4);
+    r[0] = mirrorPair<0x1B>(r[0], r[1], lane & 2);
+    r[0] += dppMove<0xB1>(r[0]);
+    r[0] = swapAdd16(r[0]);
+    if (live && lq < 16 && !(lq & 1)) A.rhs[(long long)c * 8 + (lq >> 1)] = r[0];
+  }
+  if (DMAT) {
+    __syncthreads();
+    // both cells of the wavefront in turn: O = G^T N G, 24 x 24
+    const int i = lane & 15, kk = lane >> 4;
+    f64x4 acc[2][2][2];
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      const double* g = GS + (long long)(2 * wave + z) * kSstQ * kPad;
+      const double* n = NS + (2 * wave + z) * kSstQ;
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[z][x][y] = f64x4{0, 0, 0, 0};
+      const int i1 = 16 + (i & 7);  // rows 24..31 of the second tile repeat 16..23 and are not used
+#pragma unroll
+      for (int k0 = 0; k0 < kSstQ; k0 += 4) {
+        const double* gk = g + (k0 + kk) * kPad;
+        const double nk = n[k0 + kk], b0 = gk[i], b1 = gk[i1];
+        const double a0 = nk * b0, a1 = nk * b1;
+        acc[z][0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[z][0][0], 0, 0, 0);
+        acc[z][0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[z][0][1], 0, 0, 0);
+        acc[z][1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[z][1][0], 0, 0, 0);
+        acc[z][1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[z][1][1], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+    // the products replace the gradients: row p of a cell at p * kPad
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      double* O = GS + (long long)(2 * wave + z) * kSstQ * kPad;
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int p = 16 * x + kk + 4 * r, q = 16 * y + i;
+            if (p < kComp && q < kComp) O[p * kPad + q] = acc[z][x][y][r];
+          }
+    }
+    __syncthreads();
     const int a = lane >> 3, b = lane & 7;
-    double z = 0.0;
-    for (int q = 0; q < kSstQ; ++q) {
-      const double gd = GP[wv][q][a][0] * GP[wv][q][b][0] + GP[wv][q][a][1] * GP[wv][q][b][1] +
-                        GP[wv][q][a][2] * GP[wv][q][b][2];
-      z += DW[wv][q] * gd + RW[wv][q] * PH[wv][q][a] * PH[wv][q][b];
-    }
-    mat[(long long)c * 64 + lane] = conv ? z + conv[(long long)c * 64 + lane] : z;
-    if (dmat) {
-      double* Dm = dmat + ((long long)c * 64 + lane) * 9;
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) {
-          double v = 0.0;
-          for (int q = 0; q < kSstQ; ++q)
-            v += NW[wv][q] * (GP[wv][q][a][j] * GP[wv][q][b][i] - (2.0 / 3.0) * GP[wv][q][a][i] * GP[wv][q][b][j]);
-          Dm[3 * i + j] = v;
-        }
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      const int cz = blockIdx.x * 8 + 2 * wave + z;
+      if (cz >= A.nc) break;
+      const double* O = GS + (long long)(2 * wave + z) * kSstQ * kPad;
+      double* D = A.dmat + ((long long)cz * 64 + lane) * 9;
+      for (int ii = 0; ii < 3; ++ii)
+        for (int j = 0; j < 3; ++j)
+          D[3 * ii + j] = O[(3 * a + j) * kPad + 3 * b + ii] - (2.0 / 3.0) * O[(3 * a + ii) * kPad + 3 * b + j];
     }
   }
-  if (rhs && lane < 8) {
-    double z = 0.0;
-    for (int q = 0; q < kSstQ; ++q) z += SW[wv][q] * PH[wv][q][lane];
-    rhs[(long long)c * 8 + lane] = z;
-  }
+}
+
+inline void launchSstVolume(hipStream_t s, const SstVolArgs& A) {
+  if (A.dmat) hipLaunchKernelGGL((k_sst_volume<true>), (A.nc + 7) / 8, 256, 0, s, A);
+  else hipLaunchKernelGGL((k_sst_volume<false>), (A.nc + 7) / 8, 256, 0, s, A);
+  NODALS_LAUNCHED();
 }
 
 }  // namespace dev

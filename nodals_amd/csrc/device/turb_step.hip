@@ -208,11 +208,14 @@ int H8Solver::turbEquation(int eq, double* rel0, double* rel1) {
   const TurbConsts K{S_.pipe.R, S_.pipe.nu, P.kFloor, P.omegaFloor, P.deviatoric ? 1 : 0, eq};
   double* x = eq == 0 ? st.k.data() : st.w.data();
   // element blocks: volume terms with the molecular diffusion, plus convection
-  hipLaunchKernelGGL(k_sst_volume, (nc_ + 3) / 4, 256, 0, s, nc_, cref_.data(), cinvJ_.data(), cdet_.data(),
-                     sstXY_.data(), u_.data(), fixedVal_.data(), st.k.data(), st.k.data(), st.w.data(), st.w.data(),
-                     sstQuad_.data(), S_.pipe.R, S_.pipe.nu, eq, P.kFloor, P.omegaFloor, P.deviatoric ? 1 : 0,
-                     st.blk.data(), st.brhs.data(), st.sref.data(), S_.pipe.nu, st.conv.data(), st.vdistPtr());
-  NODALS_LAUNCHED();
+  {
+    SstVolArgs A = turbVolArgs(eq);
+    A.mat = st.blk.data();
+    A.rhs = st.brhs.data();
+    A.nuBase = S_.pipe.nu;
+    A.conv = st.conv.data();
+    launchSstVolume(s, A);
+  }
   if (T.nInlet > 0) {
     hipLaunchKernelGGL(k_turb_inlet, (T.nInlet + 3) / 4, 256, 0, s, T.nInlet, st.fcell.data(), st.flf.data(),
                        st.fgeom.data(), cref_.data(), st.sref.data(), cinvJ_.data(), sstXY_.data(), u_.data(),
@@ -363,13 +366,10 @@ void H8Solver::turbCouple(bool on) {
 // blocks of the convection (cbuf_), which the momentum gather then
 // assembles like the convection itself (Dirichlet columns to the rhs).
 void H8Solver::eddyDiffusion() {
-  TurbState& st = *turb_;
-  const TurbParams& P = st.P;
-  hipLaunchKernelGGL(k_sst_volume, (nc_ + 3) / 4, 256, 0, stream_, nc_, cref_.data(), cinvJ_.data(), cdet_.data(),
-                     sstXY_.data(), u_.data(), fixedVal_.data(), st.k.data(), st.k.data(), st.w.data(), st.w.data(),
-                     sstQuad_.data(), S_.pipe.R, S_.pipe.nu, 2, P.kFloor, P.omegaFloor, P.deviatoric ? 1 : 0,
-                     cbuf_.data(), nullptr, st.sref.data(), 0.0, cbuf_.data(), st.vdistPtr());
-  NODALS_LAUNCHED();
+  SstVolArgs A = turbVolArgs(2);
+  A.mat = cbuf_.data();
+  A.conv = cbuf_.data();
+  launchSstVolume(stream_, A);
 }
 
 std::vector<double> H8Solver::turbField(const std::string& n) {

@@ -253,12 +253,13 @@ void H8Solver::wallAssemble() {
   // convection (skew or advective) and the eddy-viscosity blocks, plus the
   // deviatoric tensors
   convLocal(s, 8192);
-  hipLaunchKernelGGL(k_sst_volume, (nc_ + 3) / 4, 256, 0, s, nc_, cref_.data(), cinvJ_.data(), cdet_.data(),
-                     sstXY_.data(), u_.data(), fixedVal_.data(), st.k.data(), st.k.data(), st.w.data(), st.w.data(),
-                     sstQuad_.data(), S_.pipe.R, S_.pipe.nu, 2, TP.kFloor, TP.omegaFloor, TP.deviatoric ? 1 : 0,
-                     cbuf_.data(), nullptr, st.sref.data(), 0.0, cbuf_.data(), st.vdistPtr(),
-                     w.P.deviatoric ? w.dbuf.data() : nullptr);
-  NODALS_LAUNCHED();
+  {
+    SstVolArgs V = turbVolArgs(2);
+    V.mat = cbuf_.data();
+    V.conv = cbuf_.data();
+    V.dmat = w.P.deviatoric ? w.dbuf.data() : nullptr;
+    launchSstVolume(s, V);
+  }
   if (nf > 0) {
     hipLaunchKernelGGL(k_wall_fit, blocksFor(nf), 256, 0, s, nf, w.wn.data(), w.qw.data(), w.bp.data(),
                        w.wcell.data(), cref_.data(), u_.data(), fixedVal_.data(), st.scell.data(), st.sphi.data(),
