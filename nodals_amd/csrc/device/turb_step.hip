@@ -228,10 +228,14 @@ int H8Solver::turbEquation(int eq, double* rel0, double* rel1) {
   if (eq == 1 && T.nWallQ > 0) {
     const WallConsts W{P.wallGamma, P.ofKappa,     P.ofE, P.ofBeta1, P.ofReBlend, P.ofProdLimit,
                        T.heights[4] - T.heights[0], st.omegaFitPoints, P.omegaMode};
-    hipLaunchKernelGGL(k_turb_wall_coef, blocksFor(T.nWallQ), 256, 0, s, T.nWallQ, st.wgeom.data(), st.scell.data(),
-                       st.sl.data(), st.sphi.data(), st.sy.data(), cref_.data(), st.sref.data(), cinvJ_.data(), sstXY_.data(),
-                       u_.data(), fixedVal_.data(), st.k.data(), st.w.data(), K, W, tri12(), st.coef.data(),
-                       st.target.data(), st.counters.data() + 2, st.vdistPtr(), st.mu.data());
+#define NODALS_WALL_COEF(LN)                                                                                        \
+  hipLaunchKernelGGL(k_turb_wall_coef<LN>, blocksFor((long long)T.nWallQ * LN), 256, 0, s, T.nWallQ, st.wgeom.data(), \
+                     st.scell.data(), st.sl.data(), st.sphi.data(), st.sy.data(), cref_.data(), st.sref.data(),       \
+                     cinvJ_.data(), sstXY_.data(), u_.data(), fixedVal_.data(), st.k.data(), st.w.data(), K, W,       \
+                     tri12(), st.coef.data(), st.target.data(), st.counters.data() + 2, st.vdistPtr(), st.mu.data())
+    if (st.omegaFitPoints >= 3) NODALS_WALL_COEF(kFitLanes);
+    else NODALS_WALL_COEF(1);
+#undef NODALS_WALL_COEF
     NODALS_LAUNCHED();
     if (P.omegaMode == 2)
       hipLaunchKernelGGL(k_turb_wall_trace, (T.nWallQ + 3) / 4, 256, 0, s, T.nWallQ, st.wcell.data(), st.wlf.data(),
