@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(256) k_dense_mv(int n, int ld, const TV* __res
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    s[r] = groupSum(s[r], 64);
+    s[r] = laneSum<64>(s[r]);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][r] = s[r];
   }
   __syncthreads();

@@ -67,17 +67,26 @@ static __global__ void __launch_bounds__(256) k_conv_local(int nc, const int* __
 // nonzeros) and face-bubble rows (about 12).  One launch covers both: blocks
 // [0, nbLong) give each long row LL lanes, the remaining blocks give each
 // short row LS lanes, so neither class runs a long serial loop nor leaves
-// most lanes idle.  The branch is uniform per block.
-#define NODALS_TWO_CLASS(LL, LS, nLong, nShort, nbLong, BODY)            \
-  if ((int)blockIdx.x < (nbLong)) {                                       \
-    const int gid_ = blockIdx.x * 256 + threadIdx.x;                      \
-    const int q_ = gid_ / (LL);                                           \
-    if (q_ < (nLong)) BODY(LL, q_, gid_ % (LL), true);                   \
-  } else {                                                                \
-    const int gid_ = ((int)blockIdx.x - (nbLong)) * 256 + threadIdx.x;    \
-    const int q_ = gid_ / (LS);                                           \
-    if (q_ < (nShort)) BODY(LS, q_, gid_ % (LS), false);                 \
+// most lanes idle.  The branch is uniform per block.  Both classes' blocks are
+// padded to a multiple of eight and dealt so that each XCD takes one
+// contiguous eighth of either class (within a colour, whose rows are in mesh
+// order, the eighths of both classes gather the same region).  With the sums
+// in registers a colour pass went from 5.6 to 5.2 us on the 40k pipe and from
+// 128 to 122 us on the 769k one.  Class lists sorted over the colours by mesh
+// position made k_mom_rows slower (738 -> 978 us at 769k: its rows' own arrays
+// are in colour order).
+#define NODALS_TWO_CLASS(LL, LS, nLong, nShort, nbLong, BODY)                                      \
+  if ((int)blockIdx.x < (nbLong)) {                                                                 \
+    const int gid_ = xcdBlock((int)blockIdx.x, (nbLong)) * 256 + (int)threadIdx.x;                  \
+    const int q_ = gid_ / (LL);                                                                     \
+    if (q_ < (nLong)) BODY(LL, q_, gid_ % (LL), true);                                             \
+  } else {                                                                                          \
+    const int gid_ =                                                                                \
+        xcdBlock((int)blockIdx.x - (nbLong), (int)gridDim.x - (nbLong)) * 256 + (int)threadIdx.x;   \
+    const int q_ = gid_ / (LS);                                                                     \
+    if (q_ < (nShort)) BODY(LS, q_, gid_ % (LS), false);                                           \
   }
+inline int classBlocks(long long rows, int lanes) { return xcdGrid(blocksFor(rows * lanes)); }
 
 // Per momentum row: gather the assembled matrix (persistent diffusion +
 // convection terms), row-L1 under-relaxation delta = (1/alpha-1) sum|a_ik|
@@ -94,7 +103,7 @@ struct MomRowsArgs {
   const double* fixedVal;
   const int* incOff;
   const unsigned* incPacked;
-  const double *bcoef, *p, *srhs, *u;
+  const double *incB, *p, *srhs, *u;  // incB[k][3]: B of incidence entry k
   double fac;
   double *aval, *delta, *diag, *rau, *brhs;
 };
@@ -124,8 +133,8 @@ __device__ __forceinline__ void mom_row(const MomRowsArgs& A, int i, int lane) {
     sabs += fabs(v);
     if (k == dp) vdiag = v;
   }
-  sabs = groupSum(sabs, L);
-  vdiag = groupSum(vdiag, L);
+  sabs = laneSum<L>(sabs);
+  vdiag = laneSum<L>(vdiag);
   const double de = A.fac * sabs;
   const double dg = vdiag + de;
   double c0 = 0, c1 = 0, c2 = 0;
@@ -139,19 +148,18 @@ __device__ __forceinline__ void mom_row(const MomRowsArgs& A, int i, int lane) {
   double t0 = 0, t1 = 0, t2 = 0;
   for (int k = A.incOff[i] + lane; k < A.incOff[i + 1]; k += L) {
     const unsigned pk = A.incPacked[k];
-    const int c = (int)(pk >> 3), a = (int)(pk & 7u);
-    const double pv = A.p[c];
-    const double* B = A.bcoef + (long long)c * 24 + 3 * a;
+    const double pv = A.p[pk >> 3];
+    const double* B = A.incB + 3ll * k;
     t0 += B[0] * pv;
     t1 += B[1] * pv;
     t2 += B[2] * pv;
   }
-  c0 = groupSum(c0, L);
-  c1 = groupSum(c1, L);
-  c2 = groupSum(c2, L);
-  t0 = groupSum(t0, L);
-  t1 = groupSum(t1, L);
-  t2 = groupSum(t2, L);
+  c0 = laneSum<L>(c0);
+  c1 = laneSum<L>(c1);
+  c2 = laneSum<L>(c2);
+  t0 = laneSum<L>(t0);
+  t1 = laneSum<L>(t1);
+  t2 = laneSum<L>(t2);
   if (dp >= rb + lane && ((dp - rb - lane) % L) == 0) A.aval[dp] = dg;
   if (lane == 0) {
     A.delta[i] = de;
@@ -224,9 +232,9 @@ __device__ __forceinline__ void mom_gs_row(int i, int lane, const int* __restric
       }
     }
   }
-  s0 = groupSum(s0, L);
-  s1 = groupSum(s1, L);
-  s2 = groupSum(s2, L);
+  s0 = laneSum<L>(s0);
+  s1 = laneSum<L>(s1);
+  s2 = laneSum<L>(s2);
   if (lane == 0) {
     const double iv = 1.0 / dg;
     const double w1 = 1.0 - omega;
@@ -291,9 +299,9 @@ __device__ __forceinline__ void mom_norm_row(int i, int lane, const int* __restr
       }
     }
   }
-  s0 = groupSum(s0, L);
-  s1 = groupSum(s1, L);
-  s2 = groupSum(s2, L);
+  s0 = laneSum<L>(s0);
+  s1 = laneSum<L>(s1);
+  s2 = laneSum<L>(s2);
   if (lane == 0) {
     acc[0] += b0 * b0;
     acc[1] += b1 * b1;
@@ -319,7 +327,7 @@ __global__ void __launch_bounds__(256) k_mom_norms(int nLong, const int* __restr
   // all six sums with cross-lane shuffles per wavefront, one barrier
 #pragma unroll
   for (int q = 0; q < 6; ++q) {
-    const double t = groupSum(acc[q], 64);
+    const double t = laneSum<64>(acc[q]);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][q] = t;
   }
   __syncthreads();
@@ -333,38 +341,36 @@ __global__ void __launch_bounds__(256) k_mom_norms(int nLong, const int* __restr
 // the pressure right-hand side, with block partials of r^2.  A pinned cell
 // (pin >= 0, closed domains) gets a zero right-hand side; its residual still
 // counts in the norm.
-static __global__ void __launch_bounds__(256) k_continuity(int nc, const int* __restrict__ cref,
-                                                    const double* __restrict__ bcoef,
-                                                    const double* __restrict__ fixedDiv, const double* __restrict__ u,
-                                                    int pin, double* __restrict__ negCont, double* __restrict__ part) {
-  __shared__ double sh[4];
+//
+// Eight lanes per cell, lane = basis, so the references and B are read
+// contiguously; blocks of sixteen wavefronts, because the fixed
+// kReduceParts blocks have to fill the chip.
+constexpr int kContThreads = 1024;
+static __global__ void __launch_bounds__(kContThreads) k_continuity(
+    int nc, const int* __restrict__ cref, const double* __restrict__ bcoef, const double* __restrict__ fixedDiv,
+    const double* __restrict__ u, int pin, double* __restrict__ negCont, double* __restrict__ part) {
+  __shared__ double sh[kContThreads / 64];
+  const int a = threadIdx.x & 7;
   double acc = 0.0;
-  for (int c = blockIdx.x * 256 + threadIdx.x; c < nc; c += gridDim.x * 256) {
-    double s = fixedDiv[c];
-    const double* B = bcoef + (long long)c * 24;
-    // all eight gathers are issued before the sum (a fixed DOF reads DOF 0,
-    // in bounds, and is not accumulated); the sum keeps the basis order
-    int gq[8];
-    double xq[24];
-#pragma unroll
-    for (int a = 0; a < 8; ++a) gq[a] = cref[(long long)c * 8 + a];
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const long long g = gq[a] < 0 ? 0 : gq[a];
-      xq[3 * a] = u[3 * g];
-      xq[3 * a + 1] = u[3 * g + 1];
-      xq[3 * a + 2] = u[3 * g + 2];
+  for (int c = (blockIdx.x * kContThreads + threadIdx.x) >> 3; c < nc; c += gridDim.x * (kContThreads / 8)) {
+    const int g = cref[(long long)c * 8 + a];
+    const double* B = bcoef + (long long)c * 24 + 3 * a;
+    const double b0 = B[0], b1 = B[1], b2 = B[2], f = fixedDiv[c];
+    double s = 0.0;
+    if (g >= 0) s = b0 * u[3ll * g] + b1 * u[3ll * g + 1] + b2 * u[3ll * g + 2];
+    s = f + laneSum<8>(s);
+    if (a == 0) {
+      negCont[c] = c == pin ? 0.0 : -s;
+      acc += s * s;
     }
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const double t = B[3 * a] * xq[3 * a] + B[3 * a + 1] * xq[3 * a + 1] + B[3 * a + 2] * xq[3 * a + 2];
-      if (gq[a] >= 0) s += t;
-    }
-    negCont[c] = c == pin ? 0.0 : -s;
-    acc += s * s;
   }
-  acc = blockSum256(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = acc;
+  acc = laneSum<64>(acc);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const double t = laneSum<16>(sh[threadIdx.x & 15]);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
+  }
 }
 
 // W[c][a] = rAU_g B[c][a] for the free DOF g of cell c's basis a (zero for
@@ -420,7 +426,7 @@ __global__ void __launch_bounds__(256) k_fine_refresh(
       }
     }
     if (L1) {
-      sabs = groupSum(sabs, L);
+      sabs = laneSum<L>(sabs);
       if (lane == 0) {
         l1d[c] = sabs;
         if (F32 || B16) l1f[c] = (float)sabs;

@@ -551,6 +551,14 @@ void H8Solver::upload() {
   }
   incOff_.upload(ioff);
   incPacked_.upload(ipk);
+  {
+    std::vector<double> ib(ipk.size() * 3);
+    for (std::size_t k = 0; k < ipk.size(); ++k)
+      for (int d = 0; d < 3; ++d)
+        ib[3 * k + (std::size_t)d] = S_.bcoef[(std::size_t)(ipk[k] >> 3) * 24 + 3 * (ipk[k] & 7u) + (std::size_t)d];
+    if (ib.empty()) ib.push_back(0.0);
+    incB_.upload(ib);
+  }
 
   // state vectors
   auto aos = [&](const std::array<std::vector<double>, 3>& v) {
@@ -741,7 +749,7 @@ void H8Solver::assemble(double alphaU, double rauScale, bool convReady) {
   a.fixedVal = fixedVal_.data();
   a.incOff = incOff_.data();
   a.incPacked = incPacked_.data();
-  a.bcoef = bcoef_.data();
+  a.incB = incB_.data();
   a.p = p_.data();
   a.srhs = srhs_.data();
   a.u = u_.data();
@@ -751,7 +759,7 @@ void H8Solver::assemble(double alphaU, double rauScale, bool convReady) {
   a.diag = diag_.data();
   a.rau = rau_.data();
   a.brhs = brhs_.data();
-  const int nbL = blocksFor((long long)nLong_ * kLongLanes), nbS = blocksFor((long long)nShort_ * kShortLanes);
+  const int nbL = classBlocks(nLong_, kLongLanes), nbS = classBlocks(nShort_, kShortLanes);
   hipLaunchKernelGGL((k_mom_rows<kLongLanes, kShortLanes>), nbL + nbS, 256, 0, stream_, a, nLong_, longRows_.data(),
                      nShort_, shortRows_.data(), nbL);
   NODALS_LAUNCHED();
@@ -777,7 +785,7 @@ const char* H8Solver::momentumWork(const std::string& mode, double omega, int ou
       const int r0 = colorOff_[(std::size_t)c], r1 = colorOff_[(std::size_t)c + 1];
       if (r1 <= r0) continue;
       const int rs = colorSplit_[(std::size_t)c];
-      const int nbL = blocksFor((long long)(rs - r0) * kLongLanes), nbS = blocksFor((long long)(r1 - rs) * kShortLanes);
+      const int nbL = classBlocks((rs - r0), kLongLanes), nbS = classBlocks((r1 - rs), kShortLanes);
       if (probeOn_ && probeKind_ == 2) {  // timed from its own dispatch packet
         hipExtLaunchKernelGGL((k_mom_gs<kLongLanes, kShortLanes>), dim3(nbL + nbS), dim3(256), 0, stream_,
                               probeEv_[2 * (std::size_t)probeUsed_], probeEv_[2 * (std::size_t)probeUsed_ + 1], 0, r0,
@@ -831,7 +839,7 @@ const char* H8Solver::momentumWork(const std::string& mode, double omega, int ou
 
 void H8Solver::momentumAuditLaunch(double* out) {
   requireDevice();
-  const int nbL = blocksFor((long long)nLong_ * kNormLongLanes), nbS = blocksFor((long long)nShort_ * kNormShortLanes);
+  const int nbL = classBlocks(nLong_, kNormLongLanes), nbS = classBlocks(nShort_, kNormShortLanes);
   const int grid = nbL + nbS;
   if (normPart_.size() < (std::size_t)grid * 6) normPart_.alloc((std::size_t)grid * 6);
   hipLaunchKernelGGL((k_mom_norms<kNormLongLanes, kNormShortLanes>), grid, 256, 0, stream_, nLong_, longRows_.data(),
@@ -861,7 +869,7 @@ std::array<double, 3> H8Solver::momentumAuditRead(const double* h) {
 void H8Solver::continuityLaunch(double* out) {
   requireDevice();
   double* part = red_.partials();
-  hipLaunchKernelGGL(k_continuity, kReduceParts, 256, 0, stream_, nc_, cref_.data(), bcoef_.data(), fixedDiv_.data(),
+  hipLaunchKernelGGL(k_continuity, kReduceParts, kContThreads, 0, stream_, nc_, cref_.data(), bcoef_.data(), fixedDiv_.data(),
                      u_.data(), S_.pinCell, cont_.data(), part);
   NODALS_LAUNCHED();
   hipLaunchKernelGGL(k_reduce_final, 1, 256, 0, stream_, kReduceParts, part, out);
@@ -1670,7 +1678,7 @@ double H8Solver::timeKernel(const std::string& kernel, int reps, double* bytes) 
     by = 16.0 * (double)n;
   } else if (kernel == "continuity") {
     launch = [this]() {
-      hipLaunchKernelGGL(k_continuity, kReduceParts, 256, 0, stream_, nc_, cref_.data(), bcoef_.data(),
+      hipLaunchKernelGGL(k_continuity, kReduceParts, kContThreads, 0, stream_, nc_, cref_.data(), bcoef_.data(),
                          fixedDiv_.data(), u_.data(), S_.pinCell, cont_.data(), red_.partials());
       NODALS_LAUNCHED();
     };

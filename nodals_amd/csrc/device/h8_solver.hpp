@@ -316,6 +316,7 @@ class H8Solver {
   DBuf<double> cinvJ_, cdet_, bcoef_, fixedVal_, centT_;
   DBuf<int> mrow_, mcol_, mdiagPos_, termOff_, termIdx_, fixOff_, fixTerm_, incOff_;
   DBuf<unsigned> incPacked_;
+  DBuf<double> incB_;  // B of every incidence entry, in incidence order
   DBuf<double> mdiff_, aval_, cbuf_;
   DBuf<double> u_, brhs_, srhs_, delta_, diag_, rau_, rauSnap_;
   DBuf<double> p_, fixedDiv_, cont_, pcx_;

@@ -128,7 +128,7 @@ static __global__ void __launch_bounds__(256) k_gs_update_dots(long long n, int 
   {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     for (int q = 0; q < k; ++q) {
-      const double v = groupSum(0.0 + partIn[(long long)q * kReduceParts + threadIdx.x], 64);
+      const double v = laneSum<64>(0.0 + partIn[(long long)q * kReduceParts + threadIdx.x]);
       if (lane == 0) sh[wv][q] = v;
     }
     __syncthreads();
@@ -161,7 +161,7 @@ static __global__ void __launch_bounds__(256) k_gs_update_dots(long long n, int 
 #pragma unroll
   for (int q = 0; q < 33; ++q) {
     if (q < k || q == 32) {
-      const double t = groupSum(sv[q], 64);
+      const double t = laneSum<64>(sv[q]);
       if (lane == 0) sh[wv][q] = t;
     }
   }
@@ -238,7 +238,7 @@ static __global__ void __launch_bounds__(256) k_arnoldi_update(long long n, int 
   for (int q = wv; q <= j + 1; q += 4) {
     double v = 0.0;
     for (int i = lane; i < nparts; i += 64) v += part[(long long)q * nparts + i];
-    v = groupSum(v, 64);
+    v = laneSum<64>(v);
     if (lane == 0) h2s[q] = v;
   }
   const bool lead = blockIdx.x == 0;

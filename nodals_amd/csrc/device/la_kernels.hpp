@@ -3,8 +3,9 @@
 // Row-parallel kernels map one row to a group of LANES consecutive lanes of
 // a wavefront (LANES in {4,8,16,32,64}), chosen from the mean row length so a
 // 64-lane wavefront keeps its loads coalesced on short rows without idling on
-// long ones.  Group reductions use __shfl_xor inside the group, so every row's
-// sum has a fixed order: results are deterministic run to run.  Global FP64
+// long ones.  Group reductions are cross-lane moves inside the group
+// (laneSum), so every row's sum has a fixed order: results are deterministic run
+// to run.  Global FP64
 // reductions are two-stage (fixed grid of partial sums, then one block per
 // output), also deterministic.  Nothing here uses atomics.
 #pragma once
@@ -15,12 +16,6 @@ namespace nodals {
 namespace dev {
 
 constexpr int kReduceParts = 256;  // partial sums per reduction (grid size)
-
-template <class T>
-__device__ __forceinline__ T groupSum(T v, int lanes) {
-  for (int o = lanes >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, lanes);
-  return v;
-}
 
 // Sum over groups of L consecutive lanes (every lane gets it) with cross-lane
 // moves inside the registers: quad swaps, half-row and row mirrors (the
@@ -50,6 +45,14 @@ __device__ __forceinline__ double swapAdd16(double v) {
   const auto l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
   const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
   return fromWords(l[0], h[0]) + fromWords(l[1], h[1]);
+}
+__device__ __forceinline__ int swapAdd16(int v) {
+  const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+  return (int)(r[0] + r[1]);
+}
+__device__ __forceinline__ int swapAdd32(int v) {
+  const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+  return (int)(r[0] + r[1]);
 }
 __device__ __forceinline__ float swapAdd32(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -168,9 +171,8 @@ __device__ __forceinline__ TS rowDot(int k0, int e, const int* __restrict__ col,
 // by the next from the same L2.  A bijection on [0, gridDim.x): blocks past
 // the rows exit in the caller's bounds check, whatever the hardware's
 // placement.
-__device__ __forceinline__ int xcdRowBlock() {
-  return (int)(blockIdx.x & 7u) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
-}
+__device__ __forceinline__ int xcdBlock(int block, int grid) { return (block & 7) * (grid >> 3) + (block >> 3); }
+__device__ __forceinline__ int xcdRowBlock() { return xcdBlock((int)blockIdx.x, (int)gridDim.x); }
 inline int xcdGrid(int grid) { return (grid + 7) & ~7; }
 
 // ---------------------------------------------------------------- BLAS-1
@@ -250,7 +252,7 @@ static __global__ void __launch_bounds__(256) k_multi_axpy_dev(long long n, int 
 }
 // ---------------------------------------------------------------- reductions
 __device__ __forceinline__ double blockSum256(double v, double* sh) {
-  v = groupSum(v, 64);
+  v = laneSum<64>(v);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) sh[w] = v;
   __syncthreads();
@@ -293,7 +295,7 @@ __global__ void __launch_bounds__(256) k_multidot_part(long long n, int k, const
 #pragma unroll
   for (int j = 0; j <= KMAX; ++j) {
     if (j < k || (NORM && j == KMAX)) {
-      const double t = groupSum(s[j], 64);
+      const double t = laneSum<64>(s[j]);
       if (lane == 0) sh[wv][j] = t;
     }
   }
@@ -325,7 +327,7 @@ __global__ void __launch_bounds__(256) k_spmv(int n, const int* __restrict__ row
   if (r >= n) return;
   TV s = rowDot<LANES, TV>(
       row[r] + lane, row[r + 1], col, -1, [&](int k) { return ld<TV>(val, k); }, [&](int j) { return x[j]; });
-  s = groupSum(s, LANES);
+  s = laneSum<LANES>(s);
   if (lane == 0) {
     if (RESID) y[r] = b[r] - s;
     else if (ACC) y[r] += s;
@@ -347,7 +349,7 @@ __global__ void __launch_bounds__(256) k_schur_spmv(int n, const int* __restrict
   if (r >= n) return;
   double s = rowDot<LANES, double>(
       row[r] + lane, row[r + 1], col, -1, [&](int k) { return val[k]; }, [&](int j) { return x[j]; });
-  s = groupSum(s, LANES);
+  s = laneSum<LANES>(s);
   if (lane == 0) y[r] = s;
 }
 
@@ -371,7 +373,7 @@ __global__ void __launch_bounds__(256) k_jacobi_pre_resid(int n, const int* __re
   TV s = rowDot<LANES, TV>(
       row[i] + lane, row[i + 1], col, -1, [&](int k) { return ld<TV>(val, k); },
       [&](int j) { return (TV)omega * (TV)b[j] / d[j]; });
-  s = groupSum(s, LANES);
+  s = laneSum<LANES>(s);
   if (lane == 0) {
     const TV bi = (TV)b[i];
     t[i] = (TV)omega * bi / d[i];
@@ -393,7 +395,7 @@ __global__ void __launch_bounds__(256) k_resid_jacobi_post(int n, const int* __r
   if (i >= n) return;
   TV s = rowDot<LANES, TV>(
       row[i] + lane, row[i + 1], col, -1, [&](int k) { return ld<TV>(val, k); }, [&](int j) { return t[j]; });
-  s = groupSum(s, LANES);
+  s = laneSum<LANES>(s);
   if (lane == 0) {
     const TV r = (TV)b[i] - s;
     z[i] = (TZ)(t[i] + (TV)omega * r / d[i]);
@@ -422,7 +424,7 @@ __global__ void __launch_bounds__(256) k_resid_jacobi_post_agg(
   TV s = rowDot<LANES, TV>(
       row[i] + lane, row[i + 1], col, -1, [&](int k) { return ld<TV>(val, k); },
       [&](int j) { return t[j] + mulRn(pval[j], xc[pcol[j]]); });
-  s = groupSum(s, LANES);
+  s = laneSum<LANES>(s);
   if (lane == 0) {
     const TV ti = t[i] + mulRn(pval[i], xc[pcol[i]]);
     const TV r = (TV)b[i] - s;
@@ -443,7 +445,7 @@ __global__ void __launch_bounds__(256) k_row_l1(int n, const int* __restrict__ r
     const TV v = ld<TV>(val, k);
     s += v >= TV(0) ? v : -v;
   }
-  s = groupSum(s, LANES);
+  s = laneSum<LANES>(s);
   if (lane == 0) l1[r] = s;
 }
 

@@ -347,10 +347,10 @@ static __global__ void __launch_bounds__(256) k_turb_gather(
     const int tm = rhsTerm[t];
     if (tm < rhsLimit) rs += brhs[tm];
   }
-  l1 = groupSum(l1, L);
-  d0 = groupSum(d0, L);
-  rs = groupSum(rs, L);
-  const int nonFinite = groupSum(finite ? 0 : 1, L);
+  l1 = laneSum<L>(l1);
+  d0 = laneSum<L>(d0);
+  rs = laneSum<L>(rs);
+  const int nonFinite = laneSum<L>(finite ? 0 : 1);
   if (lane == 0) {
     const double delta = (1.0 / alpha - 1.0) * l1, dn = d0 + delta;
     if (nonFinite || !(l1 > 0.0) || !isfinite(delta) || !(dn > 0.0) || !isfinite(dn)) {

@@ -213,7 +213,7 @@ struct WallRowsArgs {
   const double* fixedVal;
   const int* incOff;
   const unsigned* incPacked;
-  const double *bcoef, *p, *srhs, *u;
+  const double *incB, *p, *srhs, *u;
   double fac, rauScale;
   double *K, *brhs, *rau3, *r3, *delta3, *diag3;
   int* bad;
@@ -269,11 +269,11 @@ __device__ __forceinline__ void wall_row(const WallRowsArgs& A, int i, int lane)
       }
   }
   for (int d = 0; d < 3; ++d) {
-    l1[d] = groupSum(l1[d], L);
-    l1p[d] = groupSum(l1p[d], L);
-    dg[d] = groupSum(dg[d], L);
-    dpn[d] = groupSum(dpn[d], L);
-    ddev[d] = groupSum(ddev[d], L);
+    l1[d] = laneSum<L>(l1[d]);
+    l1p[d] = laneSum<L>(l1p[d]);
+    dg[d] = laneSum<L>(dg[d]);
+    dpn[d] = laneSum<L>(dpn[d]);
+    ddev[d] = laneSum<L>(ddev[d]);
   }
   // Dirichlet columns: convection (+ eddy diffusion) and deviatoric terms
   double c3[3] = {0, 0, 0};
@@ -289,14 +289,13 @@ __device__ __forceinline__ void wall_row(const WallRowsArgs& A, int i, int lane)
   double t3[3] = {0, 0, 0};
   for (int k = A.incOff[i] + lane; k < A.incOff[i + 1]; k += L) {
     const unsigned pk = A.incPacked[k];
-    const int c = (int)(pk >> 3), a = (int)(pk & 7u);
-    const double pv = A.p[c];
-    const double* B = A.bcoef + (long long)c * 24 + 3 * a;
+    const double pv = A.p[pk >> 3];
+    const double* B = A.incB + 3ll * k;
     for (int d = 0; d < 3; ++d) t3[d] += B[d] * pv;
   }
   for (int d = 0; d < 3; ++d) {
-    c3[d] = groupSum(c3[d], L);
-    t3[d] = groupSum(t3[d], L);
+    c3[d] = laneSum<L>(c3[d]);
+    t3[d] = laneSum<L>(t3[d]);
   }
   // the lane that wrote the diagonal entry's block relaxes it
   if (dp >= rb + lane && ((dp - rb - lane) % L) == 0)
@@ -419,9 +418,9 @@ __device__ __forceinline__ void m3_row(int i, int lane, const int* __restrict__ 
     s1 += Kk[3] * x0 + Kk[4] * x1 + Kk[5] * x2;
     s2 += Kk[6] * x0 + Kk[7] * x1 + Kk[8] * x2;
   }
-  s0 = groupSum(s0, L);
-  s1 = groupSum(s1, L);
-  s2 = groupSum(s2, L);
+  s0 = laneSum<L>(s0);
+  s1 = laneSum<L>(s1);
+  s2 = laneSum<L>(s2);
   if (lane != 0) return;
   double r[3] = {b[3ll * i] - s0, b[3ll * i + 1] - s1, b[3ll * i + 2] - s2};
   const double* Kd = K + 9ll * mdiagPos[i];
@@ -456,15 +455,10 @@ __global__ void __launch_bounds__(256) k_m3_gs(int r0, int rs, int r1, int nbLon
                                                const double* __restrict__ K, const double* __restrict__ b,
                                                double* __restrict__ x, const int* __restrict__ bubFace,
                                                const double* __restrict__ wn, double omega, int* __restrict__ bad) {
-  if ((int)blockIdx.x < nbLong) {
-    const int gid = blockIdx.x * 256 + threadIdx.x;
-    const int i = r0 + gid / LL;
-    if (i < rs) m3_row<LL>(i, gid % LL, mrow, mcol, mdiagPos, K, b, x, bubFace, wn, omega, bad);
-  } else {
-    const int gid = ((int)blockIdx.x - nbLong) * 256 + threadIdx.x;
-    const int i = rs + gid / LS;
-    if (i < r1) m3_row<LS>(i, gid % LS, mrow, mcol, mdiagPos, K, b, x, bubFace, wn, omega, bad);
-  }
+#define NODALS_M3_BODY(LN, q, lane, isLong) \
+  m3_row<LN>((isLong) ? r0 + (q) : rs + (q), lane, mrow, mcol, mdiagPos, K, b, x, bubFace, wn, omega, bad)
+  NODALS_TWO_CLASS(LL, LS, rs - r0, r1 - rs, nbLong, NODALS_M3_BODY)
+#undef NODALS_M3_BODY
 }
 
 // bn[f] = n_f . v[bubble_f] (v interleaved [nv][3]).
@@ -525,38 +519,49 @@ static __global__ void k_wall_t(int nf, const int* __restrict__ bub, const int* 
 // bubble of face f (a wall bubble's incidence is its one cell).
 static __global__ void k_i3_bn(int nf, const int* __restrict__ bub, const double* __restrict__ wn,
                                const int* __restrict__ incOff, const unsigned* __restrict__ incPacked,
-                               const double* __restrict__ bcoef, const double* __restrict__ x,
+                               const double* __restrict__ incB, const double* __restrict__ x,
                                double* __restrict__ bn) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= nf) return;
   const int i = bub[f];
   double w[3] = {0, 0, 0};
   for (int k = incOff[i]; k < incOff[i + 1]; ++k) {
-    const unsigned pk = incPacked[k];
-    const int c = (int)(pk >> 3), a = (int)(pk & 7u);
-    const double* B = bcoef + (long long)c * 24 + 3 * a;
-    for (int d = 0; d < 3; ++d) w[d] += B[d] * x[c];
+    const double xc = x[incPacked[k] >> 3];
+    for (int d = 0; d < 3; ++d) w[d] += incB[3ll * k + d] * xc;
   }
   bn[f] = wn[3 * f] * w[0] + wn[3 * f + 1] * w[1] + wn[3 * f + 2] * w[2];
 }
 
-// Stage 2, one thread per free DOF: y = Q R (T^T (B^T x)), R = diag(r3).
-static __global__ void k_i3_dof(int nv, const int* __restrict__ incOff, const unsigned* __restrict__ incPacked,
-                                const double* __restrict__ bcoef, const double* __restrict__ x,
-                                const double* __restrict__ r3, const int* __restrict__ wallDof,
-                                const int* __restrict__ dofOff, const int* __restrict__ dofFace,
-                                const unsigned char* __restrict__ isBub, const double* __restrict__ wn,
-                                const double* __restrict__ bn, double* __restrict__ y) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nv) return;
+// Stage 2: y = Q R (T^T (B^T x)), R = diag(r3), per free DOF.  Vertex DOFs
+// (about 24 cells) take eight lanes, face bubbles (two cells) one thread; B is
+// read in incidence order, so a row's entries are one contiguous run.  One
+// thread a DOF gathering B from the cells' table took 73 us at 207k cells,
+// this 21 us (it moves about 110 MB).
+template <int L>
+__device__ __forceinline__ void i3_dof_row(int i, int lane, const int* __restrict__ incOff,
+                                           const unsigned* __restrict__ incPacked, const double* __restrict__ incB,
+                                           const double* __restrict__ x, const double* __restrict__ r3,
+                                           const int* __restrict__ wallDof, const int* __restrict__ dofOff,
+                                           const int* __restrict__ dofFace, const unsigned char* __restrict__ isBub,
+                                           const double* __restrict__ wn, const double* __restrict__ bn,
+                                           double* __restrict__ y) {
   double w[3] = {0, 0, 0};
-  for (int k = incOff[i]; k < incOff[i + 1]; ++k) {
-    const unsigned pk = incPacked[k];
-    const int c = (int)(pk >> 3), a = (int)(pk & 7u);
-    const double* B = bcoef + (long long)c * 24 + 3 * a;
-    for (int d = 0; d < 3; ++d) w[d] += B[d] * x[c];
+  const int ke = incOff[i + 1], t = wallDof[i];
+  for (int k0 = incOff[i] + lane; k0 < ke; k0 += 4 * L) {
+    double xc[4], B[4][3];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = min(k0 + q * L, ke - 1);
+      xc[q] = x[incPacked[k] >> 3];
+      for (int d = 0; d < 3; ++d) B[q][d] = incB[3ll * k + d];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (k0 + q * L < ke)
+        for (int d = 0; d < 3; ++d) w[d] += B[q][d] * xc[q];
   }
-  const int t = wallDof[i];
+  for (int d = 0; d < 3; ++d) w[d] = laneSum<L>(w[d]);
+  if (lane != 0) return;
   int bf = -1;
   if (t >= 0) {
     if (isBub[t]) {
@@ -578,30 +583,49 @@ static __global__ void k_i3_dof(int nv, const int* __restrict__ incOff, const un
   for (int d = 0; d < 3; ++d) y[3ll * i + d] = w[d];
 }
 
-// Stage 3, one thread per cell: out = B (T y); the wall bubbles of the
-// cell's wall faces are taken at their T-constrained values.
-static __global__ void k_i3_cell(int nc, const int* __restrict__ cref, const double* __restrict__ bcoef,
-                                 const double* __restrict__ y, const int* __restrict__ cellWallOff,
-                                 const int* __restrict__ cellWall, const int* __restrict__ wlf,
-                                 const int* __restrict__ bub, const int* __restrict__ vert,
-                                 const double* __restrict__ wn, double* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+constexpr int kI3Lanes = 8;
+static __global__ void __launch_bounds__(256) k_i3_dof(
+    int nLong, const int* __restrict__ longRows, int nShort, const int* __restrict__ shortRows, int nbLong,
+    const int* __restrict__ incOff, const unsigned* __restrict__ incPacked, const double* __restrict__ incB,
+    const double* __restrict__ x, const double* __restrict__ r3, const int* __restrict__ wallDof,
+    const int* __restrict__ dofOff, const int* __restrict__ dofFace, const unsigned char* __restrict__ isBub,
+    const double* __restrict__ wn, const double* __restrict__ bn, double* __restrict__ y) {
+#define NODALS_I3_BODY(LN, q, lane, isLong)                                                                          \
+  i3_dof_row<LN>((isLong) ? longRows[q] : shortRows[q], lane, incOff, incPacked, incB, x, r3, wallDof, dofOff, dofFace, \
+                 isBub, wn, bn, y)
+  NODALS_TWO_CLASS(kI3Lanes, 1, nLong, nShort, nbLong, NODALS_I3_BODY)
+#undef NODALS_I3_BODY
+}
+
+// Stage 3, eight lanes per cell (lane = basis, so B and the references are read
+// contiguously): out = B (T y); the wall bubbles of the cell's wall faces are
+// taken at their T-constrained values.  One thread a cell took 44 us at
+// 207k cells, this under 20.
+static __global__ void __launch_bounds__(256) k_i3_cell(int nc, const int* __restrict__ cref,
+                                                        const double* __restrict__ bcoef,
+                                                        const double* __restrict__ y,
+                                                        const int* __restrict__ cellWallOff,
+                                                        const int* __restrict__ cellWall, const int* __restrict__ wlf,
+                                                        const int* __restrict__ bub, const int* __restrict__ vert,
+                                                        const double* __restrict__ wn, double* __restrict__ out) {
+  const int gid = xcdRowBlock() * 256 + (int)threadIdx.x;
+  const int c = gid >> 3, a = gid & 7;
   if (c >= nc) return;
+  const int g = cref[c * 8 + a];
   const double* B = bcoef + (long long)c * 24;
+  const int w0 = cellWallOff[c], w1 = cellWallOff[c + 1];
   double s = 0.0;
-  for (int a = 0; a < 8; ++a) {
-    const int g = cref[c * 8 + a];
-    if (g < 0) continue;
-    s += B[3 * a] * y[3ll * g] + B[3 * a + 1] * y[3ll * g + 1] + B[3 * a + 2] * y[3ll * g + 2];
-  }
-  for (int t = cellWallOff[c]; t < cellWallOff[c + 1]; ++t) {
+  if (g >= 0) s = B[3 * a] * y[3ll * g] + B[3 * a + 1] * y[3ll * g + 1] + B[3 * a + 2] * y[3ll * g + 2];
+  s = laneSum<8>(s);
+  if (a != 0) return;
+  for (int t = w0; t < w1; ++t) {
     const int f = cellWall[t];
     const double n[3] = {wn[3 * f], wn[3 * f + 1], wn[3 * f + 2]};
     const double* Yb = y + 3ll * bub[f];
     double delta = -(n[0] * Yb[0] + n[1] * Yb[1] + n[2] * Yb[2]);
     double sn = 0.0;
-    for (int a = 0; a < 3; ++a) {
-      const double* X = y + 3ll * vert[3 * f + a];
+    for (int v = 0; v < 3; ++v) {
+      const double* X = y + 3ll * vert[3 * f + v];
       sn += n[0] * X[0] + n[1] * X[1] + n[2] * X[2];
     }
     delta -= (20.0 / 27.0) * sn;

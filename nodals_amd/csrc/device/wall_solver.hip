@@ -292,7 +292,7 @@ void H8Solver::wallAssemble() {
   a.fixedVal = fixedVal_.data();
   a.incOff = incOff_.data();
   a.incPacked = incPacked_.data();
-  a.bcoef = bcoef_.data();
+  a.incB = incB_.data();
   a.p = p_.data();
   a.srhs = srhs_.data();
   a.u = u_.data();
@@ -305,7 +305,7 @@ void H8Solver::wallAssemble() {
   a.delta3 = w.delta3.data();
   a.diag3 = w.diag3.data();
   a.bad = w.counters.data() + 2;
-  const int nbL = blocksFor((long long)nLong_ * kLongLanes), nbS = blocksFor((long long)nShort_ * kShortLanes);
+  const int nbL = classBlocks(nLong_, kLongLanes), nbS = classBlocks(nShort_, kShortLanes);
   hipLaunchKernelGGL((k_wall_rows<kLongLanes, kShortLanes>), nbL + nbS, 256, 0, s, a, nLong_, longRows_.data(),
                      nShort_, shortRows_.data(), nbL);
   NODALS_LAUNCHED();
@@ -358,7 +358,7 @@ void H8Solver::wallMomentum(int sweeps, double omega, int symmetric, double* rel
       const int r0 = colorOff_[(std::size_t)c], r1 = colorOff_[(std::size_t)c + 1];
       if (r1 <= r0) continue;
       const int rs = colorSplit_[(std::size_t)c];
-      const int nbL = blocksFor((long long)(rs - r0) * kLongLanes), nbS = blocksFor((long long)(r1 - rs) * kShortLanes);
+      const int nbL = classBlocks((rs - r0), kLongLanes), nbS = classBlocks((r1 - rs), kShortLanes);
       if (probeOn_ && probeKind_ == 2) {  // the launch probe times each colour from its own dispatch packet
         hipExtLaunchKernelGGL((k_m3_gs<kLongLanes, kShortLanes>), dim3(nbL + nbS), dim3(256), 0, s,
                               probeEv_[2 * (std::size_t)probeUsed_], probeEv_[2 * (std::size_t)probeUsed_ + 1], 0,
@@ -390,14 +390,16 @@ void H8Solver::wallSchur(hipStream_t s, const double* x, double* y) {
   const int nf = w.W.nf;
   if (nf > 0) {
     hipLaunchKernelGGL(k_i3_bn, blocksFor(nf), 256, 0, s, nf, w.bub.data(), w.wn.data(), incOff_.data(),
-                       incPacked_.data(), bcoef_.data(), x, w.bn.data());
+                       incPacked_.data(), incB_.data(), x, w.bn.data());
     NODALS_LAUNCHED();
   }
-  hipLaunchKernelGGL(k_i3_dof, blocksFor(nv_), 256, 0, s, nv_, incOff_.data(), incPacked_.data(), bcoef_.data(), x,
+  const int nbI = classBlocks(nLong_, kI3Lanes);
+  hipLaunchKernelGGL(k_i3_dof, nbI + classBlocks(nShort_, 1), 256, 0, s, nLong_, longRows_.data(), nShort_,
+                     shortRows_.data(), nbI, incOff_.data(), incPacked_.data(), incB_.data(), x,
                      w.r3.data(), w.wallDof.data(), w.dofOff.data(), w.dofFace.data(), w.isBub.data(), w.wn.data(),
                      w.bn.data(), w.y3.data());
   NODALS_LAUNCHED();
-  hipLaunchKernelGGL(k_i3_cell, blocksFor(nc_), 256, 0, s, nc_, cref_.data(), bcoef_.data(), w.y3.data(),
+  hipLaunchKernelGGL(k_i3_cell, xcdGrid(blocksFor(8ll * nc_)), 256, 0, s, nc_, cref_.data(), bcoef_.data(), w.y3.data(),
                      w.cellWallOff.data(), w.cellWall.data(), w.wlf.data(), w.bub.data(), w.vert.data(), w.wn.data(),
                      y);
   NODALS_LAUNCHED();
@@ -411,10 +413,12 @@ void H8Solver::wallCorrect(const double* dp) {
   hipStream_t s = stream_;
   if (nf > 0) {
     hipLaunchKernelGGL(k_i3_bn, blocksFor(nf), 256, 0, s, nf, w.bub.data(), w.wn.data(), incOff_.data(),
-                       incPacked_.data(), bcoef_.data(), dp, w.bn.data());
+                       incPacked_.data(), incB_.data(), dp, w.bn.data());
     NODALS_LAUNCHED();
   }
-  hipLaunchKernelGGL(k_i3_dof, blocksFor(nv_), 256, 0, s, nv_, incOff_.data(), incPacked_.data(), bcoef_.data(), dp,
+  const int nbI = classBlocks(nLong_, kI3Lanes);
+  hipLaunchKernelGGL(k_i3_dof, nbI + classBlocks(nShort_, 1), 256, 0, s, nLong_, longRows_.data(), nShort_,
+                     shortRows_.data(), nbI, incOff_.data(), incPacked_.data(), incB_.data(), dp,
                      w.r3.data(), w.wallDof.data(), w.dofOff.data(), w.dofFace.data(), w.isBub.data(), w.wn.data(),
                      w.bn.data(), w.y3.data());
   NODALS_LAUNCHED();
