@@ -373,56 +373,120 @@ static __global__ void __launch_bounds__(kContThreads) k_continuity(
   }
 }
 
-// W[c][a] = rAU_g B[c][a] for the free DOF g of cell c's basis a (zero for
-// fixed ones): every term of the fine Schur refresh is then W[c][a].B[c2][b]
-// with no per-term rAU gather.
-static __global__ void k_fine_weights(int nc, const int* __restrict__ cref, const double* __restrict__ bcoef,
-                                      const double* __restrict__ rau, double* __restrict__ W) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nc * 8) return;
-  const int g = cref[t];
-  const double r = g >= 0 ? rau[g] : 0.0;
-  for (int d = 0; d < 3; ++d) W[3ll * t + d] = r * bcoef[3ll * t + d];
+// Terms of one nonzero (c, c2) of the fine Schur matrix in one word: up to
+// four (basis of c, basis of c2) pairs of six bits and their count; cells of
+// a conforming tetrahedral mesh share one vertex, an edge (2), or a face (3
+// vertices and its bubble).  Unused pairs repeat the first.  The diagonal
+// (every basis with itself; fixed ones have weight 0) and lists of other
+// lengths, which stay in the term list, have their own counts.
+constexpr unsigned kFineDiag = 7u, kFineList = 6u;
+inline unsigned packFineTerms(const unsigned* term, int count, bool diag) {
+  if (diag) return kFineDiag << 24;
+  if (count < 1 || count > 4) return kFineList << 24;
+  unsigned w = (unsigned)count << 24;
+  for (int t = 0; t < 4; ++t) w |= (term[t < count ? t : 0] & 63u) << (6 * t);
+  return w;
 }
 
-// Fine P0 Schur numeric refresh (L lanes per row, the grid looping over the
-// rows), one nonzero per lane:
-//   val[k] = sum_{shared free DOF g} rAU_g * (B[c][a] . B[c2][b])
-//          = sum (W[c][a] . B[c2][b])
+// Fine P0 Schur numeric refresh (kFineLanes lanes per row, the grid looping
+// over the rows):
+//   val[k] = sum_{shared free DOF g} rAU_g (B[c][a] . B[c2][b])
 // (h8_fine_csr_refresh_warp_kernel, h8_precomputed_b.cuh:37-91, restated as
-// a gather over the terms recorded at setup; no atomics).  Also writes the
-// diagonal, optional lower-precision copies and the row-L1 sums.  With a
-// pinned cell (pin >= 0) the off-diagonal entries of its row and column are
-// zero.
-template <int L, bool F32, bool B16, bool L1>
+// a gather; no atomics), with rAU per component (rau3) on the wall path.  The
+// row's weighted basis rAU_g B[c][a] is formed once into LDS.  A lane loads
+// the columns and packed terms of its U nonzeros, then two B vectors of each
+// (they lie in the neighbour's 192 bytes), then sums; the third and fourth
+// pair of a face neighbour follow.  Also writes the diagonal, optional
+// lower-precision copies and the row-L1 sums.  With a pinned cell (pin >= 0)
+// the off-diagonal entries of its row and column are zero.
+// Bound by latency and by the 20 bytes a nonzero that it streams: 545 us at
+// 769k cells and 30.0 us at 40k, against 1,159 and 63.3 us with offsets, a
+// term list behind them and a separate pass for the weights; with the
+// diagonal's eight products and the third and fourth pairs in run-time loops,
+// which held the other lanes of the row, 903 and 51.7 us.
+constexpr int kFineLanes = 16;  // per row; 32: 28.3 and 552 us
+template <bool F32, bool B16, bool L1>
 __global__ void __launch_bounds__(256) k_fine_refresh(
     int nc, const int* __restrict__ frow, const int* __restrict__ fcol, const int* __restrict__ fdiagPos,
-    const int* __restrict__ nzOff, const unsigned* __restrict__ nzTerm, const double* __restrict__ bcoef,
-    const double* __restrict__ W, int pin, double* __restrict__ val, float* __restrict__ valf,
+    const unsigned* __restrict__ pack, const int* __restrict__ nzOff, const unsigned* __restrict__ nzTerm,
+    const int* __restrict__ cref, const double* __restrict__ bcoef, const double* __restrict__ rau,
+    const double* __restrict__ rau3, int pin, double* __restrict__ val, float* __restrict__ valf,
     bf16* __restrict__ valb, double* __restrict__ diag, float* __restrict__ diagf, double* __restrict__ l1d,
     float* __restrict__ l1f) {
-  const int lane = threadIdx.x % L;
-  for (int c = (blockIdx.x * 256 + threadIdx.x) / L; c < nc; c += gridDim.x * (256 / L)) {
+  constexpr int L = kFineLanes, U = 5, kRows = 256 / L;  // a row has 60 to 75 nonzeros
+  __shared__ double Ws[kRows][25];
+  const int lane = threadIdx.x % L, slot = threadIdx.x / L;
+  double* W = Ws[slot];
+  for (int c = xcdRowBlock() * kRows + slot; c < nc; c += gridDim.x * kRows) {
     const int rb = frow[c], re = frow[c + 1], dp = fdiagPos[c];
-    const double* Wc = W + (long long)c * 24;
+    double dsum = 0.0;  // the diagonal: sum rAU B.B over the row's own bases
+    for (int e = lane; e < 24; e += L) {
+      const int g = cref[8ll * c + e / 3];
+      const double r = g < 0 ? 0.0 : rau3 ? rau3[3ll * g + e % 3] : rau[g];
+      const double be = bcoef[24ll * c + e], we = r * be;
+      W[e] = we;
+      dsum += we * be;
+    }
+    dsum = laneSum<L>(dsum);
+    // the row's lanes are in one wavefront: order its LDS accesses only
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
     double sabs = 0.0;
-    for (int k = rb + lane; k < re; k += L) {
-      const int c2 = fcol[k];
-      const double* Bn = bcoef + (long long)c2 * 24;
-      double v = 0.0;
-      for (int t = nzOff[k]; t < nzOff[k + 1]; ++t) {
-        const unsigned q = nzTerm[t];
-        const int a = (int)((q >> 3) & 7u), b = (int)(q & 7u);
-        v += Wc[3 * a] * Bn[3 * b] + Wc[3 * a + 1] * Bn[3 * b + 1] + Wc[3 * a + 2] * Bn[3 * b + 2];
+    for (int k0 = rb + lane; k0 < re; k0 += U * L) {
+      int c2[U];
+      unsigned pk[U];
+      double b0[U][3], b1[U][3];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = min(k0 + u * L, re - 1);
+        c2[u] = fcol[k];
+        pk[u] = pack[k];
       }
-      if ((c == pin || c2 == pin) && c != c2) v = 0.0;
-      val[k] = v;
-      if (F32) valf[k] = (float)v;
-      if (B16) valb[k] = floatToBf16((float)v);
-      if (L1) sabs += fabs(v);
-      if (k == dp) {
-        diag[c] = v;
-        if (F32 || B16) diagf[c] = (float)v;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const double* Bn = bcoef + 24ll * c2[u];
+        for (int d = 0; d < 3; ++d) {
+          b0[u][d] = Bn[3 * (pk[u] & 7u) + d];
+          b1[u][d] = Bn[3 * ((pk[u] >> 6) & 7u) + d];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u * L;
+        if (k >= re) continue;
+        const unsigned n = pk[u] >> 24;
+        const double* Bn = bcoef + 24ll * c2[u];
+        double v = 0.0;
+        auto add = [&](int a, double x, double y, double z) { v += W[3 * a] * x + W[3 * a + 1] * y + W[3 * a + 2] * z; };
+        if (n <= 4u) {
+          add((int)((pk[u] >> 3) & 7u), b0[u][0], b0[u][1], b0[u][2]);
+          if (n > 1u) add((int)((pk[u] >> 9) & 7u), b1[u][0], b1[u][1], b1[u][2]);
+          if (n > 2u) {
+            const double* B2 = Bn + 3 * ((pk[u] >> 12) & 7u);
+            const double* B3 = Bn + 3 * ((pk[u] >> 18) & 7u);
+            const double x2 = B2[0], y2 = B2[1], z2 = B2[2], x3 = B3[0], y3 = B3[1], z3 = B3[2];
+            add((int)((pk[u] >> 15) & 7u), x2, y2, z2);
+            if (n > 3u) add((int)((pk[u] >> 21) & 7u), x3, y3, z3);
+          }
+        } else if (n == kFineDiag) {
+          v = dsum;
+        } else {
+          for (int t = nzOff[k]; t < nzOff[k + 1]; ++t) {
+            const unsigned q = nzTerm[t];
+            const double* B = Bn + 3 * (q & 7u);
+            add((int)((q >> 3) & 7u), B[0], B[1], B[2]);
+          }
+        }
+        if ((c == pin || c2[u] == pin) && c != c2[u]) v = 0.0;
+        val[k] = v;
+        if (F32) valf[k] = (float)v;
+        if (B16) valb[k] = floatToBf16((float)v);
+        if (L1) sabs += fabs(v);
+        if (k == dp) {
+          diag[c] = v;
+          if (F32 || B16) diagf[c] = (float)v;
+        }
       }
     }
     if (L1) {
@@ -432,6 +496,7 @@ __global__ void __launch_bounds__(256) k_fine_refresh(
         if (F32 || B16) l1f[c] = (float)sabs;
       }
     }
+    __builtin_amdgcn_wave_barrier();  // this row's reads of W before the next row's writes
   }
 }
 

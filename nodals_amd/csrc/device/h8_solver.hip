@@ -637,21 +637,26 @@ void H8Solver::upload() {
   frow_.upload(F_.row);
   fcol_.upload(F_.col);
   fdiagPos_.upload(F_.diagPos);
-  nzOff_.upload(F_.nzOff);
-  std::vector<unsigned> nt(F_.nzTerm.size());
-  for (std::size_t t = 0; t < nt.size(); ++t) {
-    const unsigned q = F_.nzTerm[t];
-    nt[t] = ((unsigned)pinv_[(std::size_t)(q >> 6)] << 6) | (q & 63u);
+  {
+    std::vector<unsigned> pk((std::size_t)fineNnz_);
+    bool listed = false;
+    for (int c = 0; c < nc_; ++c)
+      for (int k = F_.row[(std::size_t)c]; k < F_.row[(std::size_t)c + 1]; ++k) {
+        const int t0 = F_.nzOff[(std::size_t)k], n = F_.nzOff[(std::size_t)k + 1] - t0;
+        pk[(std::size_t)k] = packFineTerms(F_.nzTerm.data() + t0, n, k == F_.diagPos[(std::size_t)c]);
+        listed = listed || pk[(std::size_t)k] >> 24 == kFineList;
+      }
+    finePack_.upload(pk);
+    if (listed) {
+      nzOff_.upload(F_.nzOff);
+      nzTerm_.upload(std::vector<unsigned>(F_.nzTerm.begin(), F_.nzTerm.end()));
+    }
   }
-  nzTerm_.upload(nt);
   fval_.alloc((std::size_t)fineNnz_);
   fdiag_.alloc((std::size_t)nc_);
   fl1_.alloc((std::size_t)nc_);
   fineMeanRow_ = (double)fineNnz_ / std::max(nc_, 1);
   fineLanes_ = lanesFor(fineMeanRow_, nc_);
-  // the refresh does ~1.5 dependent term loads per nonzero: wider groups
-  refreshLanes_ = fineNnz_ > 48ll * nc_ ? 32 : 16;
-  fineW_.alloc((std::size_t)nc_ * 24);
   if (opt_.amgPrecision != "fp64") {
     fdiagf_.alloc((std::size_t)nc_);
     fl1f_.alloc((std::size_t)nc_);
@@ -888,49 +893,28 @@ void H8Solver::refresh() {
 }
 
 void H8Solver::refreshOn(hipStream_t s) {
-  if (rau3_)  // wall-function path: B diag(rAU_x, rAU_y, rAU_z) B^T (hxt5b_boundary.cuh:1883)
-    hipLaunchKernelGGL(k_fine_weights3, blocksFor((long long)nc_ * 8), 256, 0, s, nc_, cref_.data(), bcoef_.data(),
-                       rau3_, fineW_.data());
-  else
-    hipLaunchKernelGGL(k_fine_weights, blocksFor((long long)nc_ * 8), 256, 0, s, nc_, cref_.data(), bcoef_.data(),
-                       rau_.data(), fineW_.data());
-  NODALS_LAUNCHED();
-  // A short refresh (at most five rounds of four 256-thread blocks per CU)
-  // runs on four blocks per CU (half of a CU's wave slots), each looping
-  // over rows: it runs beside the momentum sweep, whose colour launches
-  // would otherwise wait for the full grid to drain.  On the 40k-cell pipe:
-  // 1024 blocks 0.586 s to converge, 768 0.589, 1280 0.593, 1536 0.601, the
-  // full 5040 0.605 (512 finishes after the sweep: 0.605).  A longer one
-  // outlasts the sweep when stretched and keeps its full grid: capped, the
-  // 768k-cell fixed-10 run took 7.40 against 6.82 ms per SIMPLE iteration.
-  const long long full = blocksFor((long long)nc_ * refreshLanes_), cap = 4LL * cuCount_;
-  const int grid = (int)(full <= 5 * cap ? std::min(full, cap) : full);
+  // The refresh runs beside the momentum sweep.  Its whole grid is short
+  // enough now not to hold the sweep's colours up: held to 4 blocks per CU,
+  // looping over rows, the 40k-cell case took 51.7 against 51.2 ms and the
+  // 64k-cell one 35.8 against 35.3.
+  const int grid = xcdGrid(blocksFor((long long)nc_ * kFineLanes));
   const bool f32 = opt_.amgPrecision == "fp32", b16 = opt_.amgPrecision == "bf16";
   const bool l1 = opt_.amgSmoother == "l1jacobi";
-#define NODALS_REFRESH(L, F, B, LL)                                                                                  \
-  hipLaunchKernelGGL((k_fine_refresh<L, F, B, LL>), grid, 256, 0, s, nc_, frow_.data(), fcol_.data(),               \
-                     fdiagPos_.data(), nzOff_.data(), nzTerm_.data(), bcoef_.data(), fineW_.data(), S_.pinCell,     \
-                     fval_.data(), fvalf_.data(), fvalb_.data(), fdiag_.data(), fdiagf_.data(), fl1_.data(),        \
-                     fl1f_.data())
-#define NODALS_REFRESH_P(L)                         \
-  if (f32) {                                        \
-    if (l1) NODALS_REFRESH(L, true, false, true);   \
-    else NODALS_REFRESH(L, true, false, false);     \
-  } else if (b16) {                                 \
-    if (l1) NODALS_REFRESH(L, false, true, true);   \
-    else NODALS_REFRESH(L, false, true, false);     \
-  } else {                                          \
-    if (l1) NODALS_REFRESH(L, false, false, true);  \
-    else NODALS_REFRESH(L, false, false, false);    \
+#define NODALS_REFRESH(F, B, LL)                                                                                     \
+  hipLaunchKernelGGL((k_fine_refresh<F, B, LL>), grid, 256, 0, s, nc_, frow_.data(), fcol_.data(),                   \
+                     fdiagPos_.data(), finePack_.data(), nzOff_.data(), nzTerm_.data(), cref_.data(), bcoef_.data(), \
+                     rau_.data(), rau3_, S_.pinCell, fval_.data(), fvalf_.data(), fvalb_.data(), fdiag_.data(),      \
+                     fdiagf_.data(), fl1_.data(), fl1f_.data())
+  if (f32) {
+    if (l1) NODALS_REFRESH(true, false, true);
+    else NODALS_REFRESH(true, false, false);
+  } else if (b16) {
+    if (l1) NODALS_REFRESH(false, true, true);
+    else NODALS_REFRESH(false, true, false);
+  } else {
+    if (l1) NODALS_REFRESH(false, false, true);
+    else NODALS_REFRESH(false, false, false);
   }
-  switch (refreshLanes_) {
-    case 4: NODALS_REFRESH_P(4); break;
-    case 8: NODALS_REFRESH_P(8); break;
-    case 16: NODALS_REFRESH_P(16); break;
-    case 32: NODALS_REFRESH_P(32); break;
-    default: NODALS_REFRESH_P(64); break;
-  }
-#undef NODALS_REFRESH_P
 #undef NODALS_REFRESH
   NODALS_LAUNCHED();
   if (opt_.amgSmoother == "mcgs") {  // the smoother's slots mirror the values

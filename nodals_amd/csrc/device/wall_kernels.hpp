@@ -635,16 +635,6 @@ static __global__ void __launch_bounds__(256) k_i3_cell(int nc, const int* __res
   out[c] = s;
 }
 
-// W[c][a][d] = rAU_d(g) B[c][a][d] (zero for fixed DOFs): the anisotropic
-// weights of the fine Schur refresh B diag(rAU_x, rAU_y, rAU_z) B^T.
-static __global__ void k_fine_weights3(int nc, const int* __restrict__ cref, const double* __restrict__ bcoef,
-                                       const double* __restrict__ rau3, double* __restrict__ W) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nc * 8) return;
-  const int g = cref[t];
-  for (int d = 0; d < 3; ++d) W[3ll * t + d] = g >= 0 ? rau3[3ll * g + d] * bcoef[3ll * t + d] : 0.0;
-}
-
 // Wall shear of each face from its frozen fit: the traction
 // -beta (I - n n^T) u_pic at each quadrature point, integrated:
 // out[f] = (int t_x, int t_y, int t_z, int |t|) over the face.
