@@ -769,24 +769,11 @@ int nodals_gnn_sample(nodals_gnn* g, int32_t i, float* x, float* t) {
   });
 }
 
-namespace {
-// Host rows (n x 16) into a padded device copy.
-nodals::DBuf<float> gnnRows(nodals::GnnModel& m, const float* x, int width) {
-  nodals::DBuf<float> d;
-  d.alloc((std::size_t)m.paddedRows() * width);
-  nodals::dev::fill<float>(m.stream(), (long long)m.paddedRows() * width, d.data(), 0.0f);
-  NODALS_HIP(hipMemcpyAsync(d.data(), x, sizeof(float) * (std::size_t)m.n() * width, hipMemcpyHostToDevice,
-                            m.stream()));
-  return d;
-}
-}  // namespace
-
 int nodals_gnn_forward(nodals_gnn* g, const float* x, float* y) {
   return guarded([&]() {
     auto& m = gnnOf(g);
     nodals::require(x && y, "null arrays");
-    nodals::DBuf<float> X = gnnRows(m, x, nodals::GnnModel::kIn);
-    m.forward(m.stream(), X.data(), nullptr);
+    m.forward(m.stream(), m.stageX(x), nullptr);
     NODALS_HIP(hipMemcpyAsync(y, m.outputDevice(), sizeof(float) * (std::size_t)m.n(), hipMemcpyDeviceToHost,
                               m.stream()));
     NODALS_HIP(hipStreamSynchronize(m.stream()));
@@ -797,16 +784,13 @@ int nodals_gnn_gradient(nodals_gnn* g, const float* x, const float* t, float* gr
   return guarded([&]() {
     auto& m = gnnOf(g);
     nodals::require(x && t && grad, "null arrays");
-    nodals::DBuf<float> X = gnnRows(m, x, nodals::GnnModel::kIn);
-    nodals::DBuf<float> T = gnnRows(m, t, 1);
-    nodals::DBuf<float> L;
-    L.alloc(1);
-    m.forward(m.stream(), X.data(), nullptr);
-    m.backward(m.stream(), X.data(), T.data(), L.data());
+    const float *X = m.stageX(x), *T = m.stageT(t);
+    m.forward(m.stream(), X, nullptr);
+    m.backward(m.stream(), X, T, m.lossDevice());
     float lh = 0;
     NODALS_HIP(hipMemcpyAsync(grad, m.gradDevice(), sizeof(float) * (std::size_t)m.paramCount(),
                               hipMemcpyDeviceToHost, m.stream()));
-    NODALS_HIP(hipMemcpyAsync(&lh, L.data(), sizeof(float), hipMemcpyDeviceToHost, m.stream()));
+    NODALS_HIP(hipMemcpyAsync(&lh, m.lossDevice(), sizeof(float), hipMemcpyDeviceToHost, m.stream()));
     NODALS_HIP(hipStreamSynchronize(m.stream()));
     if (loss) *loss = (double)lh / m.n();
   });

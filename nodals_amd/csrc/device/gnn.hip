@@ -16,6 +16,7 @@ using dev::copy;
 using dev::fill;
 
 namespace {
+constexpr int kBackBlocks = 512;
 inline int grid1(long long n) { return (int)((n + 255) / 256); }
 }  // namespace
 
@@ -23,7 +24,9 @@ GnnModel::GnnModel(const CellGraph& g, unsigned seed) {
   require(g.n > 0 && (int)g.off.size() == g.n + 1, "GNN graph is empty or malformed");
   n_ = g.n;
   M_ = (n_ + 31) / 32 * 32;
-  chunks_ = (M_ + kChunk - 1) / kChunk;
+  // backward: at most two blocks a CU, each over its own run of row tiles
+  static_assert(kHid == kWidth && kCat == 2 * kWidth && kIn == 16, "the kernels' shapes");
+  backGrid_ = dev::xcdGrid(std::min((M_ + kTile - 1) / kTile, kBackBlocks));
   // parameter layout (FP32 master)
   int o = 0;
   oW0_ = o;
@@ -82,22 +85,22 @@ GnnModel::GnnModel(const CellGraph& g, unsigned seed) {
   w16_.alloc((std::size_t)o16);
   wt16_.alloc((std::size_t)o16);
   const std::size_t M = (std::size_t)M_;
-  Z0_.alloc(M * kHid);
-  H0_.alloc(M * kHid);
-  for (int l = 0; l < kLayers; ++l) {
-    X_[l].alloc(M * kCat);
-    Z_[l].alloc(M * kHid);
+  for (int l = 0; l <= kLayers; ++l) {
     H_[l].alloc(M * kHid);
+    mask_[l].alloc(M * 2);
   }
+  for (int l = 0; l < kLayers; ++l) Xm_[l].alloc(M * kHid);
   y_.alloc(M);
-  dHa_.alloc(M * kHid);
-  dHb_.alloc(M * kHid);
-  dZ_.alloc(M * kHid);
-  dX_.alloc(M * kCat);
-  dy_.alloc(M);
-  part_.alloc((std::size_t)chunks_ * kCat * kHid);
+  d1_.alloc(M * kHid);
+  d2a_.alloc(M * kHid);
+  d2b_.alloc(M * kHid);
+  part_.alloc((std::size_t)backGrid_ * ((std::size_t)np_ + 1));
   lossPart_.alloc((std::size_t)grid1(M_));
   loss_.alloc(1);
+  inX_.alloc(M * kIn);  // padding rows stay zero
+  inT_.alloc(M);
+  fill<float>(stream_, (long long)M_ * kIn, inX_.data(), 0.0f);
+  fill<float>(stream_, M_, inT_.data(), 0.0f);
   NODALS_HIP(hipHostMalloc((void**)&hostLoss_, sizeof(float), hipHostMallocCoherent));
   refreshWeights(stream_);
   NODALS_HIP(hipStreamSynchronize(stream_));
@@ -109,14 +112,13 @@ GnnModel::~GnnModel() {
 }
 
 void GnnModel::refreshWeights(hipStream_t s) {
-  hipLaunchKernelGGL(k_weight_bf16, grid1(kIn * kHid), 256, 0, s, kIn, kHid, P_.data() + oW0_, w16_.data() + o16W0_,
-                     wt16_.data() + o16W0_);
+  hipLaunchKernelGGL(k_weight_bf16, grid1(np_), 256, 0, s, np_, kLayers, P_.data(), w16_.data(), wt16_.data());
   NODALS_LAUNCHED();
-  for (int l = 0; l < kLayers; ++l) {
-    hipLaunchKernelGGL(k_weight_bf16, grid1(kCat * kHid), 256, 0, s, kCat, kHid, P_.data() + oW_[l],
-                       w16_.data() + o16W_[l], wt16_.data() + o16W_[l]);
-    NODALS_LAUNCHED();
-  }
+}
+
+const float* GnnModel::stage(const float* host, int width, DBuf<float>& d) {
+  NODALS_HIP(hipMemcpyAsync(d.data(), host, sizeof(float) * (std::size_t)n_ * width, hipMemcpyHostToDevice, stream_));
+  return d.data();
 }
 
 void GnnModel::getParams(float* host) const {
@@ -135,73 +137,41 @@ void GnnModel::setParams(const float* host) {
 }
 
 void GnnModel::forward(hipStream_t s, const float* X, float* y) {
-  const int gemmGrid = (M_ / 32 + 3) / 4;
-  hipLaunchKernelGGL((k_gemm<kIn, kHid, 1>), gemmGrid, 256, 0, s, M_, X, wt16_.data() + o16W0_, P_.data() + ob0_,
-                     Z0_.data(), nullptr, H0_.data());
+  hipLaunchKernelGGL(k_encode, (M_ / 32 + 3) / 4, 256, 0, s, M_, X, wt16_.data() + o16W0_, P_.data() + ob0_,
+                     H_[0].data(), mask_[0].data());
   NODALS_LAUNCHED();
-  const float* h = H0_.data();
+  const int grid = dev::xcdGrid((M_ + kTile - 1) / kTile);
   for (int l = 0; l < kLayers; ++l) {
-    hipLaunchKernelGGL(k_concat_mean, grid1((long long)M_ * 64), 256, 0, s, M_, n_, h, off_.data(), nbr_.data(),
-                       X_[l].data());
+#define NODALS_LAYER(LAST)                                                                                            \
+  hipLaunchKernelGGL((k_layer<LAST>), grid, 256, 0, s, M_, n_, H_[l].data(), off_.data(), nbr_.data(),                \
+                     wt16_.data() + o16W_[l], P_.data() + ob_[l], Xm_[l].data(), H_[l + 1].data(),                    \
+                     mask_[l + 1].data(), P_.data() + ow_, P_.data() + obout_, X, kSkip, y_.data())
+    if (l == kLayers - 1) NODALS_LAYER(true);
+    else NODALS_LAYER(false);
+#undef NODALS_LAYER
     NODALS_LAUNCHED();
-    hipLaunchKernelGGL((k_gemm<kCat, kHid, 2>), gemmGrid, 256, 0, s, M_, X_[l].data(), wt16_.data() + o16W_[l],
-                       P_.data() + ob_[l], Z_[l].data(), h, H_[l].data());
-    NODALS_LAUNCHED();
-    h = H_[l].data();
   }
-  hipLaunchKernelGGL(k_decode, grid1(M_), 256, 0, s, M_, h, P_.data() + ow_, P_.data() + obout_, X, kSkip,
-                     y_.data());
-  NODALS_LAUNCHED();
   if (y && y != y_.data()) copy<float>(s, M_, y_.data(), y);
 }
 
 void GnnModel::backward(hipStream_t s, const float* X, const float* t, float* loss) {
-  const int gemmGrid = (M_ / 32 + 3) / 4;
-  hipLaunchKernelGGL(k_mse, grid1(M_), 256, 0, s, M_, n_, y_.data(), t, dy_.data(), lossPart_.data());
-  NODALS_LAUNCHED();
-  hipLaunchKernelGGL(k_sum_parts, 1, 256, 0, s, grid1(M_), 1, lossPart_.data(), loss);
-  NODALS_LAUNCHED();
-  // decoder
-  hipLaunchKernelGGL(k_decode_back, chunks_, 256, 0, s, M_, H_[kLayers - 1].data(), P_.data() + ow_, dy_.data(),
-                     dHa_.data(), part_.data());
-  NODALS_LAUNCHED();
-  hipLaunchKernelGGL(k_sum_parts, 1, 256, 0, s, chunks_, kHid + 1, part_.data(), grad_.data() + ow_);
-  NODALS_LAUNCHED();
-  float* dH = dHa_.data();
-  float* dHn = dHb_.data();
+  float *d2 = d2a_.data(), *d2o = d2b_.data();
+#define NODALS_BACK(MODE, L, HP, XM, W, OW, OB)                                                                       \
+  hipLaunchKernelGGL((k_layer_back<MODE>), backGrid_, 256, 0, s, M_, n_, y_.data(), t, H_[kLayers].data(),            \
+                     P_.data() + ow_, d1_.data(), d2, off_.data(), nbr_.data(), mask_[L].data(), HP, XM, W,           \
+                     d1_.data(), d2o, part_.data(), np_, OW, OB, ow_);                                                \
+  NODALS_LAUNCHED()
   for (int l = kLayers - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(k_relu_back, grid1((long long)M_ * 64), 256, 0, s, M_, n_, dH, Z_[l].data(), dZ_.data());
-    NODALS_LAUNCHED();
-    // dW_l = X_l^T dZ, db_l = colsum dZ
-    hipLaunchKernelGGL((k_gemm_wgrad<kCat, kHid>), chunks_, 256, 0, s, M_, X_[l].data(), dZ_.data(), part_.data());
-    NODALS_LAUNCHED();
-    hipLaunchKernelGGL(k_sum_parts, grid1(kCat * kHid), 256, 0, s, chunks_, kCat * kHid, part_.data(),
-                       grad_.data() + oW_[l]);
-    NODALS_LAUNCHED();
-    hipLaunchKernelGGL(k_colsum64, chunks_, 256, 0, s, M_, dZ_.data(), part_.data());
-    NODALS_LAUNCHED();
-    hipLaunchKernelGGL(k_sum_parts, 1, 256, 0, s, chunks_, kHid, part_.data(), grad_.data() + ob_[l]);
-    NODALS_LAUNCHED();
-    // dX_l = dZ W_l^T (B operand: W_l row-major = (W_l^T)^T)
-    hipLaunchKernelGGL((k_gemm<kHid, kCat, 0>), gemmGrid, 256, 0, s, M_, dZ_.data(), w16_.data() + o16W_[l], nullptr,
-                       dX_.data(), nullptr, nullptr);
-    NODALS_LAUNCHED();
-    hipLaunchKernelGGL(k_concat_mean_back, grid1((long long)M_ * 64), 256, 0, s, M_, n_, dH, dX_.data(), off_.data(),
-                       nbr_.data(), dHn);
-    NODALS_LAUNCHED();
-    std::swap(dH, dHn);
+    if (l == kLayers - 1) {
+      NODALS_BACK(kTop, l + 1, H_[l].data(), Xm_[l].data(), w16_.data() + o16W_[l], oW_[l], ob_[l]);
+    } else {
+      NODALS_BACK(kMiddle, l + 1, H_[l].data(), Xm_[l].data(), w16_.data() + o16W_[l], oW_[l], ob_[l]);
+    }
+    std::swap(d2, d2o);
   }
-  // encoder
-  hipLaunchKernelGGL(k_relu_back, grid1((long long)M_ * 64), 256, 0, s, M_, n_, dH, Z0_.data(), dZ_.data());
-  NODALS_LAUNCHED();
-  hipLaunchKernelGGL((k_gemm_wgrad<kIn, kHid>), chunks_, 256, 0, s, M_, X, dZ_.data(), part_.data());
-  NODALS_LAUNCHED();
-  hipLaunchKernelGGL(k_sum_parts, grid1(kIn * kHid), 256, 0, s, chunks_, kIn * kHid, part_.data(),
-                     grad_.data() + oW0_);
-  NODALS_LAUNCHED();
-  hipLaunchKernelGGL(k_colsum64, chunks_, 256, 0, s, M_, dZ_.data(), part_.data());
-  NODALS_LAUNCHED();
-  hipLaunchKernelGGL(k_sum_parts, 1, 256, 0, s, chunks_, kHid, part_.data(), grad_.data() + ob0_);
+  NODALS_BACK(kBottom, 0, X, nullptr, nullptr, oW0_, ob0_);
+#undef NODALS_BACK
+  hipLaunchKernelGGL(k_grad_sum, (np_ + 1 + 63) / 64, 256, 0, s, backGrid_, np_, part_.data(), grad_.data(), loss);
   NODALS_LAUNCHED();
 }
 
@@ -209,10 +179,9 @@ void GnnModel::adamStep(hipStream_t s, float lr) {
   ++adamT_;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.0f - std::pow(b1, (float)adamT_), c2 = 1.0f - std::pow(b2, (float)adamT_);
-  hipLaunchKernelGGL(k_adam, grid1(np_), 256, 0, s, np_, P_.data(), grad_.data(), m_.data(), v_.data(), lr, b1, b2,
-                     eps, c1, c2);
+  hipLaunchKernelGGL(k_adam, grid1(np_), 256, 0, s, np_, kLayers, P_.data(), grad_.data(), m_.data(), v_.data(), lr,
+                     b1, b2, eps, c1, c2, w16_.data(), wt16_.data());
   NODALS_LAUNCHED();
-  refreshWeights(s);
 }
 
 void GnnModel::reserveSamples(int capacity) {
@@ -252,7 +221,7 @@ double GnnModel::train(int epochs, float lr, unsigned seed, std::vector<double>*
       backward(stream_, sampleX(i), sampleT(i), epochLoss_.data() + q++);
       adamStep(stream_, lr);
     }
-    hipLaunchKernelGGL(k_sum_parts, 1, 256, 0, stream_, nSamples_, 1, epochLoss_.data(), loss_.data());
+    hipLaunchKernelGGL(k_sum, 1, 256, 0, stream_, nSamples_, epochLoss_.data(), loss_.data());
     NODALS_LAUNCHED();
     NODALS_HIP(hipMemcpyAsync(hostLoss_, loss_.data(), sizeof(float), hipMemcpyDeviceToHost, stream_));
     NODALS_HIP(hipStreamSynchronize(stream_));
@@ -267,9 +236,9 @@ double GnnModel::evaluate() {
   double sum = 0.0;
   for (int i = 0; i < nSamples_; ++i) {
     forward(stream_, sampleX(i), nullptr);
-    hipLaunchKernelGGL(k_mse, grid1(M_), 256, 0, stream_, M_, n_, y_.data(), sampleT(i), dy_.data(), lossPart_.data());
+    hipLaunchKernelGGL(k_sq_error, grid1(M_), 256, 0, stream_, n_, y_.data(), sampleT(i), lossPart_.data());
     NODALS_LAUNCHED();
-    hipLaunchKernelGGL(k_sum_parts, 1, 256, 0, stream_, grid1(M_), 1, lossPart_.data(), loss_.data());
+    hipLaunchKernelGGL(k_sum, 1, 256, 0, stream_, grid1(M_), lossPart_.data(), loss_.data());
     NODALS_LAUNCHED();
     NODALS_HIP(hipMemcpyAsync(hostLoss_, loss_.data(), sizeof(float), hipMemcpyDeviceToHost, stream_));
     NODALS_HIP(hipStreamSynchronize(stream_));
