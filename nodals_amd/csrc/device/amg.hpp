@@ -196,6 +196,7 @@ class DevAmg {
     }
     if (dense_ < (int)nl - 1) buildDense(H, D);
     for (DBuf<TV>* v : {&fr_, &ftmp_, &fcorr_}) v->alloc((std::size_t)fineN);
+    if (steps(true) >= 2) fx_.alloc((std::size_t)fineN);
     if (opt_.kind == "mcgs") {
       require(fineColoring != nullptr, "MCGS smoother requires a fine coloring", kErrInternal);
       fineColor_.upload(*fineColoring);
@@ -228,13 +229,16 @@ class DevAmg {
   }
 
   // z = M^{-1} b for FP64 vectors b, z, replayed from one captured graph per
-  // (b, z) pair: with the fused Jacobi cycle the FP64 <-> TV roundings happen
-  // inside its first and last kernels (identical values to separate casts);
+  // (b, z) pair: with the fused cycles the FP64 <-> TV roundings happen
+  // inside their first and last kernels (identical values to separate casts);
   // otherwise through the fixed TV buffers.  Returns false (nothing done)
-  // when the smoother is not the fused Jacobi cycle.
+  // when neither fused cycle serves the fine level.
   bool applyWide(hipStream_t s, const double* b, double* z) {
-    if (!fusedJacobi()) return false;
-    wide_.run(s, graphKey({b, z, fine_.val, fine_.diag}), [&]() { fusedCycle<double, double>(s, b, z); });
+    if (!fusedJacobi() && steps(true) < 2) return false;
+    wide_.run(s, graphKey({b, z, fine_.val, fine_.diag}), [&]() {
+      if (fusedJacobi()) fusedCycle<double, double>(s, b, z);
+      else stepCycle<double, double>(s, b, z);
+    });
     return true;
   }
 
@@ -242,6 +246,10 @@ class DevAmg {
   void apply(hipStream_t s, const TV* b, TV* z) {
     if (fusedJacobi()) {
       fusedCycle<TV, TV>(s, b, z);
+      return;
+    }
+    if (steps(true) >= 2) {
+      stepCycle<TV, TV>(s, b, z);
       return;
     }
     smoothFine(s, b, z);
@@ -256,6 +264,56 @@ class DevAmg {
   }
 
  private:
+  // Steps of the Jacobi or Chebyshev smoother on the fine (coarse) levels; 0
+  // for MCGS.
+  int steps(bool fine) const {
+    if (opt_.kind == "mcgs") return 0;
+    const int m = opt_.kind == "cheb2" ? opt_.chebDegree : fine ? opt_.jacobiFineSweeps : opt_.jacobiCoarseSweeps;
+    return std::max(m, 1);
+  }
+  double stepWeight(int k, double lambda) const {
+    if (opt_.kind == "jacobi" || opt_.kind == "l1jacobi") return opt_.jacobiOmega;
+    if (opt_.kind != "cheb2") fail("unknown AMG smoother " + opt_.kind);
+    const double lo = opt_.lambdaLowFraction * lambda;
+    require(lambda > lo && lo > 0, "Chebyshev interval invalid");
+    return 1.0 / chebRoot(lambda, lo, k, opt_.chebDegree);
+  }
+
+  // Smoothing of two and more steps before and after the coarse correction,
+  // each step one matrix pass: x = S b, r = b - A x ...
+  template <class TM, class TB>
+  void stepPre(hipStream_t s, const FineView<TM, TV>& A, int m, double lambda, const TB* b, TV* x, TV* other, TV* r) {
+    const TV* den = opt_.kind == "l1jacobi" ? A.l1 : A.diag;
+    TV *from = m % 2 == 1 ? x : other, *to = m % 2 == 1 ? other : x;  // the last step lands in x
+    hipLaunchKernelGGL((k_jacobi_zero<TV, TB>), blocksFor(A.n), 256, 0, s, A.n, stepWeight(0, lambda), b, den, from);
+    NODALS_LAUNCHED();
+    for (int k = 1; k < m; ++k, std::swap(from, to))
+      residJacobiPost<TM, TV, TB, TV>(s, A.lanes, A.n, A.row, A.col, A.val, b, den, stepWeight(k, lambda), from, to);
+    residStep<kResid, TM, TV, TB>(s, A.lanes, A.n, A.row, A.col, A.val, b, den, 0.0, from, r, (TV*)nullptr,
+                                  (const TV*)nullptr, (TV*)nullptr);
+  }
+  // ... and z = x + S (b - A x).
+  template <class TM, class TB, class TZ>
+  void stepPost(hipStream_t s, const FineView<TM, TV>& A, int m, double lambda, const TB* b, const TV* x, TV* r, TV* c,
+                TV* other, TZ* z) {
+    const TV* den = opt_.kind == "l1jacobi" ? A.l1 : A.diag;
+    residStep<kFirst, TM, TV, TB>(s, A.lanes, A.n, A.row, A.col, A.val, b, den, stepWeight(0, lambda), x, r, c,
+                                  (const TV*)nullptr, (TV*)nullptr);
+    for (int k = 1; k < m - 1; ++k, std::swap(c, other))
+      residJacobiPost<TM, TV, TV, TV>(s, A.lanes, A.n, A.row, A.col, A.val, r, den, stepWeight(k, lambda), c, other);
+    residStep<kLast, TM, TV, TV, TZ>(s, A.lanes, A.n, A.row, A.col, A.val, r, den, stepWeight(m - 1, lambda), c,
+                                     (TV*)nullptr, (TV*)nullptr, x, z);
+  }
+  template <class TB, class TZ>
+  void stepCycle(hipStream_t s, const TB* b, TZ* z) {
+    const int m = steps(true);
+    stepPre<TF>(s, fine_, m, fineLambda_, b, fx_.data(), ftmp_.data(), fr_.data());
+    restrictTo(s, P_[0], fr_.data(), L_[0].b.data());
+    vcycle(s, 0, L_[0].b.data(), L_[0].x.data());
+    prolongAdd(s, P_[0], L_[0].x.data(), fx_.data());
+    stepPost<TF>(s, fine_, m, fineLambda_, b, fx_.data(), fr_.data(), fcorr_.data(), ftmp_.data(), z);
+  }
+
   template <class TB, class TZ>
   // Pre-smoothing + residual, coarse correction, residual + post-smoothing:
   // two fine passes instead of five kernels.
@@ -511,38 +569,6 @@ class DevAmg {
     return centre - radius * std::cos(pi * (2.0 * k + 1.0) / (2.0 * degree));
   }
 
-  // Jacobi and Chebyshev smoothing of an operator (row, col, val, diag, l1)
-  // from x = 0; r is scratch.
-  template <class TM>
-  void smooth(hipStream_t s, int n, int lanes, const int* row, const int* col, const TM* val, const TV* diag,
-              const TV* l1, double lambda, int jacobiSweeps, const TV* b, TV* x, TV* r) {
-    const int grid = blocksFor(n);
-    if (opt_.kind == "jacobi" || opt_.kind == "l1jacobi") {
-      const TV* den = opt_.kind == "l1jacobi" ? l1 : diag;
-      hipLaunchKernelGGL(k_jacobi_zero<TV>, grid, 256, 0, s, n, opt_.jacobiOmega, b, den, x);
-      NODALS_LAUNCHED();
-      for (int sw = 1; sw < jacobiSweeps; ++sw) {
-        spmv<TM, TV, true, false>(s, lanes, n, row, col, val, x, b, r);
-        hipLaunchKernelGGL(k_jacobi_add<TV>, grid, 256, 0, s, n, opt_.jacobiOmega, r, den, x);
-        NODALS_LAUNCHED();
-      }
-    } else if (opt_.kind == "cheb2") {
-      const double lo = opt_.lambdaLowFraction * lambda;
-      require(lambda > lo && lo > 0, "Chebyshev interval invalid");
-      hipLaunchKernelGGL(k_jacobi_zero<TV>, grid, 256, 0, s, n, 1.0 / chebRoot(lambda, lo, 0, opt_.chebDegree), b,
-                         diag, x);
-      NODALS_LAUNCHED();
-      for (int k = 1; k < opt_.chebDegree; ++k) {
-        spmv<TM, TV, true, false>(s, lanes, n, row, col, val, x, b, r);
-        hipLaunchKernelGGL(k_jacobi_add<TV>, grid, 256, 0, s, n, 1.0 / chebRoot(lambda, lo, k, opt_.chebDegree), r,
-                           diag, x);
-        NODALS_LAUNCHED();
-      }
-    } else {
-      fail("unknown AMG smoother " + opt_.kind);
-    }
-  }
-
   // MCGS smoothing from x = 0 (no pass reads an entry of x that an earlier
   // one has not written, so x is not cleared).  A symmetric sweep's passes
   // keep the row sum of the half that does not change until the next pass.
@@ -569,13 +595,19 @@ class DevAmg {
     }
   }
 
+  // The one step of a one-step smoother, from x = 0.
+  void smoothOnce(hipStream_t s, int n, const TV* diag, const TV* l1, double lambda, const TV* b, TV* x) {
+    hipLaunchKernelGGL((k_jacobi_zero<TV, TV>), blocksFor(n), 256, 0, s, n, stepWeight(0, lambda), b,
+                       opt_.kind == "l1jacobi" ? l1 : diag, x);
+    NODALS_LAUNCHED();
+  }
+
   void smoothFine(hipStream_t s, const TV* b, TV* x) {
     if (opt_.kind == "mcgs") {
       mcgsSmooth<TF>(s, fineGs_, fineColor_, opt_.mcgsFineSweeps, fine_.diag, b, x);
       return;
     }
-    smooth<TF>(s, fine_.n, fine_.lanes, fine_.row, fine_.col, fine_.val, fine_.diag, fine_.l1, fineLambda_,
-               opt_.jacobiFineSweeps, b, x, ftmp_.data());
+    smoothOnce(s, fine_.n, fine_.diag, fine_.l1, fineLambda_, b, x);
   }
 
   void smoothLevel(hipStream_t s, Level& A, const TV* b, TV* x) {
@@ -583,8 +615,7 @@ class DevAmg {
       mcgsSmooth<TV>(s, A.gs, A.color, opt_.mcgsCoarseSweeps, A.diag.data(), b, x);
       return;
     }
-    smooth<TV>(s, A.n, A.lanes, A.row.data(), A.col.data(), A.val.data(), A.diag.data(), A.l1.data(), A.lambda,
-               opt_.jacobiCoarseSweeps, b, x, A.tmp.data());
+    smoothOnce(s, A.n, A.diag.data(), A.l1.data(), A.lambda, b, x);
   }
 
   void vcycle(hipStream_t s, int l, const TV* b, TV* x) {
@@ -609,6 +640,23 @@ class DevAmg {
       prolongAdd(s, X, C.x.data(), A.tmp.data());
       residJacobiPost<TV, TV>(s, A.lanes, A.n, A.row.data(), A.col.data(), A.val.data(), b, den, opt_.jacobiOmega,
                               A.tmp.data(), x);
+      return;
+    }
+    if (const int m = steps(false); m >= 2) {
+      FineView<TV, TV> V;
+      V.n = A.n;
+      V.lanes = A.lanes;
+      V.row = A.row.data();
+      V.col = A.col.data();
+      V.val = A.val.data();
+      V.diag = A.diag.data();
+      V.l1 = A.l1.data();
+      stepPre<TV>(s, V, m, A.lambda, b, x, A.tmp.data(), A.r.data());
+      Level& C = L_[(std::size_t)l + 1];
+      restrictTo(s, P_[(std::size_t)l + 1], A.r.data(), C.b.data());
+      vcycle(s, l + 1, C.b.data(), C.x.data());
+      prolongAdd(s, P_[(std::size_t)l + 1], C.x.data(), x);
+      stepPost<TV>(s, V, m, A.lambda, b, x, A.r.data(), A.corr.data(), A.tmp.data(), x);
       return;
     }
     smoothLevel(s, A, b, x);
@@ -640,7 +688,7 @@ class DevAmg {
   DBuf<TV> tinv_, denseT_;
   DBuf<double> sweepScratch_;  // dense set-up only
   int termN_ = 0, dense_ = 0;
-  DBuf<TV> fr_, ftmp_, fcorr_;
+  DBuf<TV> fr_, ftmp_, fcorr_, fx_;
   GraphCache graph_;
   GraphSet wide_;
 };
