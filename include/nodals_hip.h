@@ -180,7 +180,9 @@ int nodals_h8_probe(nodals_h8* h, int32_t enable, int64_t* launches, double* tot
  * built by the coarse-level steps of build_sa_hierarchy
  * (g5_sa_host.hpp:1570-1577) applied from level 0.  options: space separated
  * key=value: precision=fp64|fp32|bf16 smoother=jacobi|l1jacobi|cheb2|mcgs
- * sweeps=N omega=W order=symmetric|forward|backward terminal=N power_its=N. */
+ * sweeps=N omega=W order=symmetric|forward|backward terminal=N power_its=N.
+ * Jacobi and Chebyshev smoothers make at least one step; mcgs with sweeps
+ * below one, or an order that is none of the three, makes no pass. */
 int nodals_sys_create(int32_t n, const int64_t* row, const int32_t* col, const double* val, const char* options,
                       nodals_sys** out);
 /* Host hierarchy only (no HIP call); only nodals_sys_info/nodals_sys_get. */

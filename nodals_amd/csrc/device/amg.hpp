@@ -109,6 +109,11 @@ class DevAmg {
 
   void setup(const AmgHierarchy& H, int fineN, const SmootherOptions& o, const Coloring* fineColoring) {
     opt_ = o;
+    // A Jacobi count below one is one step; a multicolour count below one, or
+    // an order that is none of the three, makes no pass (the smoother is zero).
+    for (int* m : {&opt_.jacobiFineSweeps, &opt_.jacobiCoarseSweeps}) *m = std::max(*m, 1);
+    const bool ordered = o.mcgsOrder == "forward" || o.mcgsOrder == "backward" || o.mcgsOrder == "symmetric";
+    for (int* m : {&opt_.mcgsFineSweeps, &opt_.mcgsCoarseSweeps}) *m = ordered ? std::max(*m, 0) : 0;
     fineN_ = fineN;
     fineLambda_ = H.fineLambda;
     const std::size_t nl = H.A.size();
@@ -125,7 +130,7 @@ class DevAmg {
     // same order as in the original numbering and results are identical.
     // perm[l][new] = original row; empty = not renumbered.
     std::vector<std::vector<int>> perm(nl), inv(nl);
-    dense_ = denseLevel(H, o);
+    dense_ = denseLevel(H);
     std::vector<DenseSetupLevel> D(nl);
     for (std::size_t l = 0; l < nl; ++l) {
       const CsrD& A = H.A[l];
@@ -425,7 +430,7 @@ class DevAmg {
   // fused Jacobi cycle has four in all).  At most kDenseRows rows, 0.65 GB in
   // FP64.  nl - 1, the terminal level, when no other pays.
   static constexpr int kDenseRows = 9000;
-  int denseLevel(const AmgHierarchy& H, const SmootherOptions& o) const {
+  int denseLevel(const AmgHierarchy& H) const {
     const int nl = (int)H.A.size();
     double below = 3.0;  // us of the cycle below the level: the terminal product
     int best = nl - 1;
@@ -433,13 +438,11 @@ class DevAmg {
       const CsrD& A = H.A[(std::size_t)l];
       if (A.n > kDenseRows) break;
       double launches = 5.0;
-      if (o.kind == "mcgs") {
+      if (opt_.kind == "mcgs") {
         const Coloring C = greedyColoring(A.n, A.row.data(), A.col.data());
-        launches += 2.0 * o.mcgsCoarseSweeps * C.ncolors * (o.mcgsOrder == "symmetric" ? 2.0 : 1.0);
-      } else if (o.kind == "cheb2") {
-        launches += 2.0 * (1.0 + 2.0 * (o.chebDegree - 1)) + 2.0;
+        launches += 2.0 * opt_.mcgsCoarseSweeps * C.ncolors * (opt_.mcgsOrder == "symmetric" ? 2.0 : 1.0);
       } else if (!fusedJacobi()) {
-        launches += 2.0 * (1.0 + 2.0 * (o.jacobiCoarseSweeps - 1)) + 2.0;
+        launches += 2.0 * (1.0 + 2.0 * (steps(false) - 1)) + 2.0;
       }
       below += 2.2 * launches;
       const double product = 3.0 + (double)A.n * denseLd(A.n) * sizeof(TV) / 4.5e6;
@@ -535,15 +538,12 @@ class DevAmg {
       }
       return;
     }
-    const bool cheb = opt_.kind == "cheb2";
-    const double lo = opt_.lambdaLowFraction * A.lambda;
-    require(!cheb || (A.lambda > lo && lo > 0), "Chebyshev interval invalid");
-    const int steps = cheb ? opt_.chebDegree : opt_.jacobiCoarseSweeps;
+    const int count = steps(false);
     const double* den = opt_.kind == "l1jacobi" ? A.l1.data() : A.diag.data();
     DBuf<double>& t = sweepScratch_;
-    if (steps > 1 && t.size() < (std::size_t)A.n * m) t.alloc((std::size_t)A.n * m);
-    for (int k = 0; k < steps; ++k) {
-      const double w = cheb ? 1.0 / chebRoot(A.lambda, lo, k, opt_.chebDegree) : opt_.jacobiOmega;
+    if (count > 1 && t.size() < (std::size_t)A.n * m) t.alloc((std::size_t)A.n * m);
+    for (int k = 0; k < count; ++k) {
+      const double w = stepWeight(k, A.lambda);
       const double* r = b;
       if (k > 0) {
         hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), x, b,
@@ -570,8 +570,9 @@ class DevAmg {
   }
 
   // MCGS smoothing from x = 0 (no pass reads an entry of x that an earlier
-  // one has not written, so x is not cleared).  A symmetric sweep's passes
-  // keep the row sum of the half that does not change until the next pass.
+  // one has not written, so x is cleared only when there is no pass).  A
+  // symmetric sweep's passes keep the row sum of the half that does not change
+  // until the next pass.
   template <class TM>
   void mcgsSmooth(hipStream_t s, const GsOperator<TM>& G, const DevColoring<TV>& C, int sweeps, const TV* diag,
                   const TV* b, TV* x) {
@@ -583,6 +584,7 @@ class DevAmg {
                          other, part, zero, opt_.mcgsOmega);
       }
     };
+    if (sweeps == 0) fill<TV>(s, C.off.back(), x, TV(0));
     const bool back = opt_.mcgsOrder == "backward";
     for (int sw = 0; sw < sweeps; ++sw) {
       const bool first = sw == 0, last = sw == sweeps - 1;

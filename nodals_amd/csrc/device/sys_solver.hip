@@ -116,7 +116,7 @@ SysSolver::SysSolver(int n, const std::int64_t* row, const std::int32_t* col, co
     v.diag = diag_.data();
     v.l1 = l1_.data();
     amg64_->setFine(v, r32.data(), A_.col.data(), pfc);
-      amg64_->fineChanged(stream_);
+    amg64_->fineChanged(stream_);
   } else {
     std::vector<float> df(A_.diag.begin(), A_.diag.end()), lf(l1.begin(), l1.end());
     diagf_.upload(df);
