@@ -193,7 +193,9 @@ void nodals_sys_destroy(nodals_sys* s);
  * info[4+l] = rows of explicit level l (l < 12). */
 int nodals_sys_info(nodals_sys* s, int64_t info[16]);
 /* Host hierarchy arrays: agg<l>, P<l>_row|col|val, A<l>_row|col|val,
- * terminal_inv, level_lambda, fine_lambda. */
+ * terminal_inv, level_lambda, fine_lambda, and gs_slots (int64[3]: slots of
+ * the multicolour Gauss-Seidel layouts of the operator's entries of lower
+ * colours, of higher colours, and of both). */
 int nodals_sys_get(nodals_sys* s, const char* name, void* host, int64_t count);
 int nodals_sys_spmv(nodals_sys* s, const double* x, double* y);
 /* One preconditioner application z = M^-1 r. */

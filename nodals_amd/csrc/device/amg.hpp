@@ -578,10 +578,8 @@ class DevAmg {
                   const TV* b, TV* x) {
     auto pass = [&](const GsSlots<TM>& S, bool reverse, const TV* other, TV* part, bool zero) {
       for (int q = 0; q < C.ncolors; ++q) {
-        const int c = reverse ? C.ncolors - 1 - q : q;
-        const int begin = C.off[(std::size_t)c], count = C.off[(std::size_t)c + 1] - begin;
-        gsColour<TM, TV>(s, S.colour[(std::size_t)c], begin, count, C.rowList(), S.col.data(), S.val.data(), diag, b, x,
-                         other, part, zero, opt_.mcgsOmega);
+        gsColour<TM, TV>(s, S, reverse ? C.ncolors - 1 - q : q, C.rowList(), diag, b, x, other, part, zero,
+                         opt_.mcgsOmega);
       }
     };
     if (sweeps == 0) fill<TV>(s, C.off.back(), x, TV(0));

@@ -531,6 +531,8 @@ int nodals_sys_get(nodals_sys* h, const char* name, void* host, int64_t count) {
       copyOut(H.levelLambda, host, count);
     } else if (n == "fine_lambda") {
       copyOut(std::vector<double>{H.fineLambda}, host, count);
+    } else if (n == "gs_slots") {
+      copyOut(s.gsSlots(), host, count);
     } else if (n[0] == 'P' || n[0] == 'A') {
       const auto u = n.find('_');
       nodals::require(u != std::string::npos, "unknown field " + n);

@@ -30,105 +30,13 @@
 // with predicated slots costs 0.3-0.4 us a pass more.
 #pragma once
 
-#include <algorithm>
-#include <thread>
 #include <vector>
 
-#include "../host/h8_setup.hpp"
+#include "../host/gs_layout.hpp"
 #include "la_kernels.hpp"
 
 namespace nodals {
 namespace dev {
-
-constexpr int kGsUnroll = 8;  // most slots a lane loads before it gathers
-
-// Which off-diagonal entries of a row a GsSlots holds.
-enum class GsHalf { lower, upper, all };
-
-// Host layout of one colour's slots: first tile, lanes a row, slots a lane
-// (at most kGsUnroll, or a multiple of it).
-struct GsColour {
-  int tile = 0, L = 1, U = 1;
-};
-
-// Lanes a row for `count` rows of at most `width` entries: the fewest that
-// leave a lane at most kGsUnroll/2 slots, widened while the colour is too
-// small to give every SIMD a wavefront (2^16 threads) and a lane still holds
-// two: within 4% of the best of 1..64 lanes on every operator above.
-inline int gsLanes(int width, int count) {
-  int L = 1;
-  while (L < 64 && (width > L * (kGsUnroll / 2) || ((long long)count * L < (1 << 16) && width > 2 * L))) L *= 2;
-  return L;
-}
-
-// Tiled slots of the chosen half of a coloured CSR operator (rows of colour
-// c: rows[off[c]..off[c+1]), or those indices themselves when rows is null).
-// Colours are independent: they are counted, then filled, in parallel.
-struct GsLayout {
-  std::vector<GsColour> colour;
-  std::vector<int> col, src;  // column (-1 where unused), CSR position (-1 where unused)
-};
-
-template <class TI>
-GsLayout gsLayout(int ncolors, const std::vector<int>& off, const int* rows, const std::vector<int>& colorOf,
-                  const TI* row, const int* col, GsHalf half) {
-  GsLayout G;
-  G.colour.resize((std::size_t)ncolors);
-  auto wanted = [&](int i, int j, int c) {
-    if (j == i) return false;
-    const int cj = colorOf[(std::size_t)j];
-    return half == GsHalf::all || (half == GsHalf::lower ? cj < c : cj > c);
-  };
-  auto eachColour = [&](auto&& body) {
-    const int nt = std::max(1, std::min(ncolors, off.back() < 4096 ? 1 : hostThreads(0)));
-    std::vector<std::thread> pool;
-    for (int t = 0; t < nt; ++t)
-      pool.emplace_back([&, t]() {
-        for (int c = t; c < ncolors; c += nt) body(c, off[(std::size_t)c], off[(std::size_t)c + 1] - off[(std::size_t)c]);
-      });
-    for (std::thread& th : pool) th.join();
-  };
-  eachColour([&](int c, int b, int n) {
-    int width = 1;
-    for (int q = 0; q < n; ++q) {
-      const int i = rows ? rows[b + q] : b + q;
-      int w = 0;
-      for (TI k = row[i]; k < row[i + 1]; ++k) w += wanted(i, col[k], c) ? 1 : 0;
-      width = std::max(width, w);
-    }
-    GsColour& C = G.colour[(std::size_t)c];
-    C.L = gsLanes(width, n);
-    C.U = (width + C.L - 1) / C.L;
-    if (C.U > kGsUnroll) C.U = (C.U + kGsUnroll - 1) / kGsUnroll * kGsUnroll;
-  });
-  long long tiles = 0;
-  for (int c = 0; c < ncolors; ++c) {
-    GsColour& C = G.colour[(std::size_t)c];
-    const int n = off[(std::size_t)c + 1] - off[(std::size_t)c], per = 64 / C.L;
-    C.tile = (int)tiles;
-    tiles += (long long)((n + per - 1) / per) * C.U;
-    require(tiles < (1ll << 31), "Gauss-Seidel slots too large for int32 tile indices");
-  }
-  G.col.assign((std::size_t)tiles * 64, -1);
-  G.src.assign((std::size_t)tiles * 64, -1);
-  eachColour([&](int c, int b, int n) {
-    const GsColour& C = G.colour[(std::size_t)c];
-    const int per = 64 / C.L;
-    for (int q = 0; q < n; ++q) {
-      const int i = rows ? rows[b + q] : b + q;
-      const std::size_t at = ((std::size_t)C.tile + (std::size_t)(q / per) * C.U) * 64 + (std::size_t)(q % per) * C.L;
-      int w = 0;
-      for (TI k = row[i]; k < row[i + 1]; ++k)
-        if (wanted(i, col[k], c)) {
-          const std::size_t s = at + (std::size_t)(w / C.L) * 64 + (std::size_t)(w % C.L);
-          G.col[s] = col[k];
-          G.src[s] = (int)k;
-          ++w;
-        }
-    }
-  });
-  return G;
-}
 
 // Slot values gathered from the CSR values they mirror.
 template <class TO, class TI>
@@ -140,8 +48,8 @@ __global__ void __launch_bounds__(256) k_gs_fill(long long n, const int* __restr
   out[i] = s >= 0 ? (TO)val[s] : TO{};
 }
 
-// One colour pass over rows crow[begin + q] (begin + q without a list), q <
-// count:  s = sum of the slots, plus other[i] when given (the row sum of the
+// One pass over a class of a colour: rows crow[begin + q] (begin + q without a
+// list), q < count:  s = sum of the slots, plus other[i] when given (the row sum of the
 // other half, unchanged since it was stored),
 //   x_i <- x_i + omega ((b_i - s) / d_i - x_i)      (x_i = 0 when zero)
 // and part[i] = the slots' sum when given.  Rows of one colour do not couple.
@@ -195,13 +103,13 @@ __global__ void __launch_bounds__(256) k_gs_colour(int begin, int count, const i
 }
 
 template <int L, class TM, class TV>
-void gsColourL(hipStream_t s, const GsColour& C, int begin, int count, const int* crow, const int* col, const TM* val,
-               const TV* diag, const TV* b, TV* x, const TV* other, TV* part, bool zero, double omega) {
-  const int per = 64 / L, grid = blocksFor((long long)((count + per - 1) / per) * 64);
+void gsClassL(hipStream_t s, const GsClass& C, const int* crow, const int* col, const TM* val, const TV* diag,
+              const TV* b, TV* x, const TV* other, TV* part, bool zero, double omega) {
+  const int per = 64 / L, grid = blocksFor((long long)((C.count + per - 1) / per) * 64);
   const long long o = (long long)C.tile * 64;
-#define NODALS_GS_COLOUR(UN, CH)                                                                                      \
-  hipLaunchKernelGGL((k_gs_colour<L, UN, TM, TV>), grid, 256, 0, s, begin, count, crow, CH, col + o, val + o, diag, b, \
-                     x, other, part, zero ? 1 : 0, omega)
+#define NODALS_GS_COLOUR(UN, CH)                                                                                       \
+  hipLaunchKernelGGL((k_gs_colour<L, UN, TM, TV>), grid, 256, 0, s, C.begin, C.count, crow, CH, col + o, val + o, diag, \
+                     b, x, other, part, zero ? 1 : 0, omega)
   switch (C.U) {
     case 1: NODALS_GS_COLOUR(1, 1); break;
     case 2: NODALS_GS_COLOUR(2, 1); break;
@@ -216,30 +124,16 @@ void gsColourL(hipStream_t s, const GsColour& C, int begin, int count, const int
   NODALS_LAUNCHED();
 }
 
-template <class TM, class TV>
-void gsColour(hipStream_t s, const GsColour& C, int begin, int count, const int* crow, const int* col, const TM* val,
-              const TV* diag, const TV* b, TV* x, const TV* other, TV* part, bool zero, double omega) {
-  if (count <= 0) return;
-  switch (C.L) {
-    case 1: gsColourL<1>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-    case 2: gsColourL<2>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-    case 4: gsColourL<4>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-    case 8: gsColourL<8>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-    case 16: gsColourL<16>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-    case 32: gsColourL<32>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-    default: gsColourL<64>(s, C, begin, count, crow, col, val, diag, b, x, other, part, zero, omega); break;
-  }
-}
-
 // Device slots of one half of an operator.
 template <class TM>
 struct GsSlots {
-  std::vector<GsColour> colour;
-  DBuf<int> col, src;
+  std::vector<std::vector<GsClass>> colour;
+  DBuf<int> col, src, rows;  // rows: the layout's own list, empty unless a colour was split
   DBuf<TM> val;
   // With the operator's values when they are fixed; otherwise fill() them.
   void upload(const GsLayout& G, const TM* csr) {
     colour = G.colour;
+    rows.upload(G.rows);
     col.upload(G.col);
     if (!csr) {
       src.upload(G.src);
@@ -260,6 +154,28 @@ struct GsSlots {
     NODALS_LAUNCHED();
   }
 };
+
+// A pass over colour c: one launch, or one a class where the colour is split.
+// crow: the colouring's row list, null where colours are contiguous rows.
+template <class TM, class TV>
+void gsColour(hipStream_t s, const GsSlots<TM>& G, int c, const int* crow, const TV* diag, const TV* b, TV* x,
+              const TV* other, TV* part, bool zero, double omega) {
+  const int* list = G.rows.size() ? G.rows.data() : crow;
+  for (const GsClass& C : G.colour[(std::size_t)c]) {
+#define NODALS_GS_LANES(LN) \
+  gsClassL<LN>(s, C, list, G.col.data(), G.val.data(), diag, b, x, other, part, zero, omega)
+    switch (C.L) {
+      case 1: NODALS_GS_LANES(1); break;
+      case 2: NODALS_GS_LANES(2); break;
+      case 4: NODALS_GS_LANES(4); break;
+      case 8: NODALS_GS_LANES(8); break;
+      case 16: NODALS_GS_LANES(16); break;
+      case 32: NODALS_GS_LANES(32); break;
+      default: NODALS_GS_LANES(64); break;
+    }
+#undef NODALS_GS_LANES
+  }
+}
 
 }  // namespace dev
 }  // namespace nodals

@@ -163,6 +163,15 @@ SysSolver::~SysSolver() {
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
+std::vector<std::int64_t> SysSolver::gsSlots() const {
+  const Coloring C = greedyColoring(A_.n, A_.row.data(), A_.col.data());
+  std::vector<std::int64_t> slots;
+  for (GsHalf h : {GsHalf::lower, GsHalf::upper, GsHalf::all})
+    slots.push_back((std::int64_t)gsLayout(C.ncolors, C.offset, C.rows.data(), C.color, A_.row.data(), A_.col.data(), h)
+                        .col.size());
+  return slots;
+}
+
 void SysSolver::apply(hipStream_t s, const double* x, double* y) {
   spmv<double, double, false, false>(s, lanes_, n_, row_.data(), col_.data(), val_.data(), x, nullptr, y);
 }

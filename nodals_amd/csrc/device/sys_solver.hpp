@@ -26,6 +26,9 @@ class SysSolver {
   int levels() const { return (int)H_.A.size(); }
   const AmgHierarchy& hierarchy() const { return H_; }
   double setupHostMs() const { return setupHostMs_; }
+  // Slots of the multicolour Gauss-Seidel layouts of the operator: its
+  // entries of lower colours, of higher colours, and both.
+  std::vector<std::int64_t> gsSlots() const;
 
   std::vector<double> spmvHost(const std::vector<double>& x);
   std::vector<double> precondHost(const std::vector<double>& r);

@@ -123,7 +123,6 @@ void H8Solver::turbInit(const TurbParams& P) {
   st->rhsOff.upload(T.rhsOff);
   st->rhsTerm.upload(T.rhsTerm);
   st->crows.upload(T.coloring.rows);
-  st->colorOff = T.coloring.offset;
   std::vector<int> fc, fl;
   std::vector<double> fg;
   for (const TurbFace& f : T.inlet) {
@@ -283,12 +282,9 @@ int H8Solver::turbEquation(int eq, double* rel0, double* rel1) {
   st.sweepGraph[eq].run(s, graphKey({x, st.val.data(), st.rhs.data()}, sweeps * 4.0 + P.gsOmega), [&]() {
     auto sweep = [&](const auto& G) {
       for (int sw = 0; sw < sweeps; ++sw)
-        for (int c = 0; c < T.coloring.ncolors; ++c) {
-          const int b = st.colorOff[(std::size_t)c], n = st.colorOff[(std::size_t)c + 1] - b;
-          gsColour(s, G.colour[(std::size_t)c], b, n, (const int*)st.crows.data(), G.col.data(), G.val.data(),
-                   (const double*)st.diag.data(), (const double*)st.rhs.data(), x, (const double*)nullptr,
-                   (double*)nullptr, false, P.gsOmega);
-        }
+        for (int c = 0; c < T.coloring.ncolors; ++c)
+          gsColour(s, G, c, st.crows.data(), (const double*)st.diag.data(), (const double*)st.rhs.data(), x,
+                   (const double*)nullptr, (double*)nullptr, false, P.gsOmega);
     };
     if (P.sweepFp32) sweep(st.gsF);
     else sweep(st.gs);

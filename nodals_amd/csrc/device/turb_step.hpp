@@ -53,7 +53,6 @@ struct TurbState {
   dev::GsSlots<float> gsF;
   DBuf<double> resid;  // residual of a scalar_solve norm
   const double* vdistPtr() const { return vdist.size() ? vdist.data() : nullptr; }
-  std::vector<int> colorOff;
   GraphCache sweepGraph[2];  // k, omega
   hipEvent_t ev[2] = {nullptr, nullptr};
   int steps = 0;

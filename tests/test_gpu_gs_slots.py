@@ -52,3 +52,27 @@ def test_slots_match_oracle(order, sweeps, precision, tol):
     print(f"\n[gpu] slots, {order} x {sweeps}, {precision}: relative difference {err:.2e}", flush=True)
     assert err < tol
     S.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,sweeps", [("symmetric", 2), ("forward", 2), ("backward", 1)])
+def test_split_colours_match_oracle(order, sweeps):
+    """Hub rows of thousands of entries: their colours are cut into classes by
+    width, which also gives the layout a row list of its own."""
+    from nodals_amd._lib import System
+    from tests.test_gs_layout import hub_system as hubs
+
+    A = hubs(12001, 2)
+    S = System(A.indptr.astype(np.int64), A.indices.astype(np.int32), A.data,
+               f"precision=fp64 smoother=mcgs sweeps={sweeps} order={order} terminal=100")
+    widest, slots = int(np.diff(A.indptr).max()), S.get("gs_slots", 3, np.int64)
+    assert slots.max() < 1000 * widest  # the padded colours would take some 6,000 rows x 4,800 entries
+    vc = O.VCycle(S.hierarchy(), O.Smoother(kind="mcgs", mcgs_fine_sweeps=sweeps, mcgs_coarse_sweeps=sweeps,
+                                            mcgs_order=order))
+    vc.set_fine(A, A.diagonal())
+    r = np.random.default_rng(2).standard_normal(A.shape[0])
+    z, zo = S.precond(r), vc.apply(r)
+    err = float(np.linalg.norm(z - zo) / np.linalg.norm(zo))
+    print(f"\n[gpu] split colours, {order} x {sweeps}: levels {S.level_rows}, relative difference {err:.2e}", flush=True)
+    assert err < 1e-12
+    S.close()
