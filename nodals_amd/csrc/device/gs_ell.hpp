@@ -78,7 +78,6 @@ __global__ void __launch_bounds__(256) k_gs_colour(int begin, int count, const i
   const TV so = other ? other[i] : TV(0);
 #pragma unroll
   for (int u = 0; u < U; ++u) v[u] = c[u] >= 0 ? x[c[u]] : TV(0);
-  const TV inv = TV(1) / di;
   TV s = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u)
@@ -98,7 +97,7 @@ __global__ void __launch_bounds__(256) k_gs_colour(int begin, int count, const i
   s = laneSum<L>(s);
   if (lane % L == 0) {
     if (part) part[i] = s;
-    x[i] = old + (TV)omega * ((bi - (s + so)) * inv - old);
+    x[i] = old + (TV)omega * ((bi - (s + so)) / di - old);
   }
 }
 

@@ -76,3 +76,30 @@ def test_split_colours_match_oracle(order, sweeps):
     print(f"\n[gpu] split colours, {order} x {sweeps}: levels {S.level_rows}, relative difference {err:.2e}", flush=True)
     assert err < 1e-12
     S.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,tol", [("fp32", 1e-5), ("bf16", 3e-2)])
+@pytest.mark.parametrize("order", ["symmetric", "forward"])
+def test_tiny_diagonals(order, precision, tol):
+    """Rows whose diagonal is below the reciprocal of the largest FP32 number:
+    the quotient by it is finite, a product with its reciprocal is not."""
+    from nodals_amd._lib import System
+    from tests.test_gpu_sys_option_limits import weighted_laplacian
+
+    A, tiny, m = weighted_laplacian(9), 2.0 ** -130, 40
+    n = A.shape[0]
+    rng = np.random.default_rng(0)
+    link = sp.coo_matrix((np.full(m, -tiny / 2), (np.arange(m), rng.choice(n, m, replace=False))), shape=(m, n))
+    B = sp.bmat([[A, link.T], [link, sp.diags([tiny] * m)]]).tocsr()
+    B.sort_indices()
+    S = System(B.indptr.astype(np.int64), B.indices.astype(np.int32), B.data,
+               f"precision={precision} smoother=mcgs sweeps=1 order={order} terminal=100")
+    vc = O.VCycle(S.hierarchy(), O.Smoother(kind="mcgs", mcgs_order=order))
+    vc.set_fine(B, B.diagonal())
+    r = np.concatenate([rng.standard_normal(n), tiny * rng.integers(-8, 9, m) / 4.0])
+    z, zo = S.precond(r), vc.apply(r)
+    print(f"\n[gpu] tiny diagonals, {order}, {precision}", flush=True)
+    for part in (slice(0, n), slice(n, n + m)):
+        assert np.linalg.norm(z[part] - zo[part]) <= tol * np.linalg.norm(zo[part])
+    S.close()
