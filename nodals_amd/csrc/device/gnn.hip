@@ -20,6 +20,7 @@ namespace {
 // 2.5% faster on a repeated call at 40,320 rows (0.60 against 0.61 ms), but
 // touch 70 MB for the first time on a first one (1.9 against 0.7 to 1.3 ms).
 constexpr int kBackBlocks = 256;
+constexpr std::size_t kStageByNull = 512 << 10;  // bytes of a host copy from which it goes by the null stream
 inline int grid1(long long n) { return (int)((n + 255) / 256); }
 }  // namespace
 
@@ -119,8 +120,22 @@ void GnnModel::refreshWeights(hipStream_t s) {
   NODALS_LAUNCHED();
 }
 
+// The runtime stages pageable memory through a ring of its own for each
+// stream, and the first 16 MB through a new one cost 0.33 ms a MB in page
+// faults.  Large copies therefore go by the null stream, whose ring is in use
+// since the mesh was uploaded, behind the model's own work; that costs 5 us a
+// copy, which small ones do not win back.  Ten forward and gradient calls of a
+// new model: 16.8 and 11.6 -> 7.2 ms at 40,320 rows (the first alone 2.5 ->
+// 0.8), 18.6 -> 16.5 at 115,200 (6.5 -> 1.9); a later call 0.58 -> 0.59 and
+// 1.29 -> 1.30 ms.
 const float* GnnModel::stage(const float* host, int width, DBuf<float>& d) {
-  NODALS_HIP(hipMemcpyAsync(d.data(), host, sizeof(float) * (std::size_t)n_ * width, hipMemcpyHostToDevice, stream_));
+  const std::size_t bytes = sizeof(float) * (std::size_t)n_ * width;
+  if (bytes < kStageByNull) {
+    NODALS_HIP(hipMemcpyAsync(d.data(), host, bytes, hipMemcpyHostToDevice, stream_));
+  } else {
+    NODALS_HIP(hipStreamSynchronize(stream_));
+    NODALS_HIP(hipMemcpy(d.data(), host, bytes, hipMemcpyHostToDevice));
+  }
   return d.data();
 }
 
