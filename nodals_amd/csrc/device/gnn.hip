@@ -16,10 +16,10 @@ using dev::copy;
 using dev::fill;
 
 namespace {
-// Blocks of a backward kernel, and so vectors of partial gradients: 512 are
-// 2.5% faster on a repeated call at 40,320 rows (0.60 against 0.61 ms), but
-// touch 70 MB for the first time on a first one (1.9 against 0.7 to 1.3 ms).
-constexpr int kBackBlocks = 256;
+// Blocks of a backward kernel, and so vectors of partial gradients (70 MB):
+// 25 to 27 us a layer and 16 us for their sum at 40,320 rows, with 256 blocks
+// 31 to 33 and 9; a first call of a new model is as fast with either.
+constexpr int kBackBlocks = 512;
 constexpr std::size_t kStageByNull = 512 << 10;  // bytes of a host copy from which it goes by the null stream
 inline int grid1(long long n) { return (int)((n + 255) / 256); }
 }  // namespace
@@ -28,7 +28,7 @@ GnnModel::GnnModel(const CellGraph& g, unsigned seed) {
   require(g.n > 0 && (int)g.off.size() == g.n + 1, "GNN graph is empty or malformed");
   n_ = g.n;
   M_ = (n_ + 31) / 32 * 32;
-  // backward: at most one block a CU, each over its own run of row tiles
+  // backward: at most two blocks a CU, each over its own run of row tiles
   static_assert(kHid == kWidth && kCat == 2 * kWidth && kIn == 16, "the kernels' shapes");
   backGrid_ = dev::xcdGrid(std::min((M_ + kTile - 1) / kTile, kBackBlocks));
   // parameter layout (FP32 master)

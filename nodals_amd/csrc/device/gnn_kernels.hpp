@@ -16,11 +16,10 @@
 // bound by latency and memory passes: the neighbour mean is gathered straight
 // into the GEMM's tile, the backward gather into the tile that feeds both
 // gradient GEMMs, and one ReLU bit per entry replaces the pre-activations.
-// Measured at 40,320 rows: forward 76 us (6 launches), backward 134 us (6),
+// Measured at 40,320 rows: forward 74 us (5 launches), backward 134 us (6),
 // where separate mean, GEMM, mask, transposed-mean, column-sum and partial-sum
 // kernels (a forward of 11, a backward of 31 launches) took about 900 us for
-// both; a forward and a gradient call with their host copies 1.51 -> 0.61 ms
-// (the figures by kernel are those of 512 backward blocks).
+// both; a forward and a gradient call with their host copies 1.51 -> 0.60 ms.
 #pragma once
 
 #include "common.hpp"
@@ -225,8 +224,7 @@ __global__ void __launch_bounds__(256) k_layer(int M, int n, const float* __rest
 //   dZ = dH where the ReLU bit is set;  dW = [Hp | Xm]^T dZ, db = sum dZ
 //   dX = dZ W^T:  D1o = dH + dX[:, :64],  D2o = dX[:, 64:] / deg
 // kBottom is the encoder: [Hp | Xm] is the input X (M x 16) and dX not needed.
-// Registers held to half, so that two blocks fit a CU and more loads are in
-// flight: 42.7 -> 26.9 us a layer at 512 blocks.
+// Two blocks a CU need the registers held to half: 42.7 -> 26.9 us a layer.
 // D1o may be D1 (a row is read by the block that writes it), D2o not D2.
 enum { kTop, kMiddle, kBottom };
 template <int MODE>
@@ -386,7 +384,7 @@ __global__ void __launch_bounds__(256, 2) k_layer_back(
 
 // grad[i] = sum over the blocks of part[block][i], and the loss behind it:
 // four wavefronts share 64 columns' rows (fixed order).  15 us for 512 blocks'
-// 70 MB, 4.6 TB/s; the grid has 256 (the launch says why).
+// 70 MB, 4.6 TB/s.
 static __global__ void __launch_bounds__(256) k_grad_sum(int blocks, int np, const float* __restrict__ part,
                                                          float* __restrict__ grad, float* __restrict__ loss) {
   __shared__ float sh[4][64];

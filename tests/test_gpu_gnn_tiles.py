@@ -1,6 +1,6 @@
 """Network kernels at cell counts below one row tile, off the tile's and the
 padding's multiples, and above one tile per block of the backward grid
-(40,320 cells: 630 tiles of 64 rows over 256 blocks): forward, loss and
+(40,320 cells: 630 tiles of 64 rows over 512 blocks): forward, loss and
 every gradient against the oracle (test_gpu_gnn.py trains).
 
 Tolerances as in test_gpu_gnn.py: BF16 rounding of GEMM inputs that differ in
