@@ -130,7 +130,10 @@ class DevAmg {
     // same order as in the original numbering and results are identical.
     // perm[l][new] = original row; empty = not renumbered.
     std::vector<std::vector<int>> perm(nl), inv(nl);
-    dense_ = denseLevel(H);
+    std::vector<Coloring> colors(nl);
+    for (std::size_t l = 0; opt_.kind == "mcgs" && l + 1 < nl; ++l)
+      colors[l] = greedyColoring(H.A[l].n, H.A[l].row.data(), H.A[l].col.data());
+    dense_ = denseLevel(H, colors);
     std::vector<DenseSetupLevel> D(nl);
     for (std::size_t l = 0; l < nl; ++l) {
       const CsrD& A = H.A[l];
@@ -138,7 +141,7 @@ class DevAmg {
       Lv.n = A.n;
       Lv.lanes = lanesFor(A.n ? (double)A.col.size() / A.n : 1.0, A.n);
       if (opt_.kind == "mcgs" && l + 1 < nl) {
-        const Coloring C = greedyColoring(A.n, A.row.data(), A.col.data());
+        const Coloring& C = colors[l];
         perm[l].assign(C.rows.begin(), C.rows.end());
         inv[l].assign((std::size_t)A.n, 0);
         for (int i = 0; i < A.n; ++i) inv[l][(std::size_t)perm[l][(std::size_t)i]] = i;
@@ -171,15 +174,21 @@ class DevAmg {
         Lv.gs.build(Lv.color.ncolors, Lv.color.off, nullptr, A.n, r32.data(), c32.data(), opt_.mcgsOrder,
                     opt_.mcgsCoarseSweeps, castVec(v64).data());
       }
-      Lv.diag.upload(castVec(d64));
-      Lv.l1.upload(castVec(l1));
-      for (DBuf<TV>* v : {&Lv.b, &Lv.x, &Lv.r, &Lv.tmp, &Lv.corr}) v->alloc((std::size_t)A.n);
+      // levelSpmv() reads the operator, x and tmp of any level; the cycle
+      // the rest, down to the right-hand side of the dense level
+      for (DBuf<TV>* v : {&Lv.x, &Lv.tmp}) v->alloc((std::size_t)A.n);
       Lv.x.upload(std::vector<TV>((std::size_t)A.n, TV(1)));
+      if ((int)l <= dense_) Lv.b.alloc((std::size_t)A.n);
+      if ((int)l < dense_) {
+        Lv.diag.upload(castVec(d64));
+        Lv.l1.upload(castVec(l1));
+        for (DBuf<TV>* v : {&Lv.r, &Lv.corr}) v->alloc((std::size_t)A.n);
+      }
       Lv.lambda = l < H.levelLambda.size() ? H.levelLambda[l] : 1.0;
       if ((int)l >= dense_) {
         D[l].n = A.n;
-        D[l].row.upload(r32);
-        D[l].col.upload(c32);
+        D[l].row = Lv.row.data();
+        D[l].col = Lv.col.data();
         D[l].val.upload(v64);
         D[l].diag.upload(d64);
         D[l].l1.upload(l1);
@@ -189,7 +198,8 @@ class DevAmg {
     }
     static const std::vector<int> none;
     for (std::size_t l = 0; l < nl; ++l)
-      uploadTransfer(H.P[l], P_[l], l > 0 ? inv[l - 1] : none, inv[l], (int)l > dense_ ? &D[l] : nullptr);
+      uploadTransfer(H.P[l], (int)l <= dense_ ? &P_[l] : nullptr, l > 0 ? inv[l - 1] : none, inv[l],
+                     (int)l > dense_ ? &D[l] : nullptr);
     termN_ = H.terminalN;
     {
       const int ld = denseLd(termN_);
@@ -352,18 +362,15 @@ class DevAmg {
   // the transpose is formed in the original numbering (within a coarse row,
   // fine rows ascend) and relabelled afterwards, so its sums keep the
   // original order too.
-  static void uploadTransfer(const Transfer& P, Xfer& X, const std::vector<int>& invF,
+  // To X for the cycle, to D in FP64 (with the coarse side's level) for the
+  // set-up of the dense operator.
+  static void uploadTransfer(const Transfer& P, Xfer* X, const std::vector<int>& invF,
                              const std::vector<int>& invC, DenseSetupLevel* D) {
-    X.nFine = P.nFine;
-    X.nCoarse = P.nCoarse;
     auto relF = [&](int i) { return invF.empty() ? i : invF[(std::size_t)i]; };
     auto relC = [&](int c) { return invC.empty() ? c : invC[(std::size_t)c]; };
     std::vector<int> origF((std::size_t)P.nFine), origC((std::size_t)P.nCoarse);
     for (int i = 0; i < P.nFine; ++i) origF[(std::size_t)relF(i)] = i;
     for (int c = 0; c < P.nCoarse; ++c) origC[(std::size_t)relC(c)] = c;
-    X.aggregation = (std::size_t)P.nFine == P.col.size();
-    for (int i = 0; X.aggregation && i < P.nFine; ++i)
-      X.aggregation = P.row[(std::size_t)i] == i && P.row[(std::size_t)i + 1] == i + 1;
     std::vector<int> pr((std::size_t)P.nFine + 1, 0), pc;
     std::vector<double> pv;
     pc.reserve(P.col.size());
@@ -376,10 +383,6 @@ class DevAmg {
       }
       pr[(std::size_t)i + 1] = (int)pc.size();
     }
-    X.prow.upload(pr);
-    X.pcol.upload(pc);
-    X.pval.upload(castVec(pv));
-    X.lanesP = lanesFor(P.nFine ? (double)P.col.size() / P.nFine : 1.0, P.nFine);
     // Transpose for gather restriction, in the original numbering.
     std::vector<int> tr((std::size_t)P.nCoarse + 1, 0);
     for (int c : P.col) ++tr[(std::size_t)c + 1];
@@ -408,10 +411,22 @@ class DevAmg {
       }
       tr2[(std::size_t)c + 1] = (int)tc2.size();
     }
-    X.trow.upload(tr2);
-    X.tcol.upload(tc2);
-    X.tval.upload(castVec(tv2));
-    if (D) {  // FP64 copies, kept with the coarse side's level
+    if (X) {
+      X->nFine = P.nFine;
+      X->nCoarse = P.nCoarse;
+      X->aggregation = (std::size_t)P.nFine == P.col.size();
+      for (int i = 0; X->aggregation && i < P.nFine; ++i)
+        X->aggregation = P.row[(std::size_t)i] == i && P.row[(std::size_t)i + 1] == i + 1;
+      X->prow.upload(pr);
+      X->pcol.upload(pc);
+      X->pval.upload(castVec(pv));
+      X->lanesP = lanesFor(P.nFine ? (double)P.col.size() / P.nFine : 1.0, P.nFine);
+      X->trow.upload(tr2);
+      X->tcol.upload(tc2);
+      X->tval.upload(castVec(tv2));
+      X->lanesT = lanesFor(P.nCoarse ? (double)P.col.size() / P.nCoarse : 1.0, P.nCoarse);
+    }
+    if (D) {
       D->prow.upload(pr);
       D->pcol.upload(pc);
       D->pval.upload(pv);
@@ -419,7 +434,6 @@ class DevAmg {
       D->tcol.upload(tc2);
       D->tval.upload(tv2);
     }
-    X.lanesT = lanesFor(P.nCoarse ? (double)tc.size() / P.nCoarse : 1.0, P.nCoarse);
   }
 
   // Coarsest-first level from which the cycle is one dense product: the
@@ -427,10 +441,15 @@ class DevAmg {
   // less than the launches it replaces (2.2 us each: with MCGS two smoothing
   // calls of a pass per colour, with the others their vector passes and
   // residuals; about five more per level for transfers and residuals; the
-  // fused Jacobi cycle has four in all).  At most kDenseRows rows, 0.65 GB in
-  // FP64.  nl - 1, the terminal level, when no other pays.
+  // fused Jacobi cycle has four in all).  nl - 1, the terminal level, when no
+  // other pays.  kDenseRows bounds what a hierarchy keeps (0.65 GB in FP64)
+  // and its set-up, not where the product pays: with MCGS and a bound of
+  // 24,000, three iterations of the wall-function loop took 362 -> 314 ms on a
+  // helix of 289k cells (12,200 rows, 1.1 GB more; FP32 333 -> 276 ms, 0.6 GB
+  // and 0.3 s of set-up more) and 453 -> 429 ms on one of 425k (17,300 rows,
+  // 2.2 GB more).
   static constexpr int kDenseRows = 9000;
-  int denseLevel(const AmgHierarchy& H) const {
+  int denseLevel(const AmgHierarchy& H, const std::vector<Coloring>& colors) const {
     const int nl = (int)H.A.size();
     double below = 3.0;  // us of the cycle below the level: the terminal product
     int best = nl - 1;
@@ -439,8 +458,8 @@ class DevAmg {
       if (A.n > kDenseRows) break;
       double launches = 5.0;
       if (opt_.kind == "mcgs") {
-        const Coloring C = greedyColoring(A.n, A.row.data(), A.col.data());
-        launches += 2.0 * opt_.mcgsCoarseSweeps * C.ncolors * (opt_.mcgsOrder == "symmetric" ? 2.0 : 1.0);
+        launches += 2.0 * opt_.mcgsCoarseSweeps * colors[(std::size_t)l].ncolors *
+                    (opt_.mcgsOrder == "symmetric" ? 2.0 : 1.0);
       } else if (!fusedJacobi()) {
         launches += 2.0 * (1.0 + 2.0 * (steps(false) - 1)) + 2.0;
       }
@@ -498,7 +517,7 @@ class DevAmg {
     }
     DenseSetupLevel& C = D[(std::size_t)l + 1];
     colsSmooth(s, A, m, A.b.data(), A.x.data());
-    hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), A.x.data(),
+    hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row, A.col, A.val.data(), A.x.data(),
                        A.b.data(), A.r.data());
     hipLaunchKernelGGL((k_cols_spmv<0>), dim3(C.n, grid.y), 256, 0, s, m, C.trow.data(), C.tcol.data(), C.tval.data(),
                        A.r.data(), nullptr, C.b.data());
@@ -506,7 +525,7 @@ class DevAmg {
     colsCycle(s, D, l + 1, m, tinv);
     hipLaunchKernelGGL((k_cols_spmv<2>), grid, 256, 0, s, m, C.prow.data(), C.pcol.data(), C.pval.data(), C.x.data(),
                        nullptr, A.x.data());
-    hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), A.x.data(),
+    hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row, A.col, A.val.data(), A.x.data(),
                        A.b.data(), A.r.data());
     NODALS_LAUNCHED();
     // the post-smoothing reads A.r and needs a residual of its own: A.b is
@@ -527,7 +546,7 @@ class DevAmg {
           const int c = reverse ? nc - 1 - q : q;
           const int begin = A.colorOff[(std::size_t)c], count = A.colorOff[(std::size_t)c + 1] - begin;
           if (count <= 0) continue;
-          hipLaunchKernelGGL(k_cols_gs, dim3(count, grid.y), 256, 0, s, m, begin, A.row.data(), A.col.data(),
+          hipLaunchKernelGGL(k_cols_gs, dim3(count, grid.y), 256, 0, s, m, begin, A.row, A.col,
                              A.val.data(), A.diag.data(), b, x, opt_.mcgsOmega);
           NODALS_LAUNCHED();
         }
@@ -546,7 +565,7 @@ class DevAmg {
       const double w = stepWeight(k, A.lambda);
       const double* r = b;
       if (k > 0) {
-        hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row.data(), A.col.data(), A.val.data(), x, b,
+        hipLaunchKernelGGL((k_cols_spmv<1>), grid, 256, 0, s, m, A.row, A.col, A.val.data(), x, b,
                            t.data());
         NODALS_LAUNCHED();
         r = t.data();

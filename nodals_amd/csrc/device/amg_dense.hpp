@@ -153,12 +153,13 @@ __global__ void __launch_bounds__(256) k_cols_store(int m, int c0, int ld, const
   T[(long long)blockIdx.x * ld + c0 + c] = (TV)x[(long long)blockIdx.x * m + c];
 }
 
-// FP64 copies of one level for the set-up of the dense operator: the
-// operator in the stored numbering, its transfers to the next level, the
-// colour ranges and the column blocks.
+// One level for the set-up of the dense operator: the operator (the level's
+// pattern in its stored numbering, FP64 values), the transfers from the next
+// finer level, the colour ranges and the column blocks.
 struct DenseSetupLevel {
   int n = 0;
-  DBuf<int> row, col, prow, pcol, trow, tcol;
+  const int *row = nullptr, *col = nullptr;
+  DBuf<int> prow, pcol, trow, tcol;
   DBuf<double> val, diag, l1, pval, tval, b, x, r, corr;
   std::vector<int> colorOff;
   double lambda = 1.0;
