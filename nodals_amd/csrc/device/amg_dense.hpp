@@ -11,12 +11,14 @@
 // the hierarchy's type, as the terminal inverse is).
 //
 // The product is bound by reading the matrix once: n^2 values at about 4.5
-// TB/s.  Measured (FP64, MCGS): three iterations of the wall-function loop
-// on the 207k-cell helix, whose CF level of 8,530 rows with the 47 + 46 colours
-// below it becomes one 582 MB product, 520 -> 364 ms; the 64^3 Poisson solve
-// (1,073 rows, 44 colours) 18.9 -> 13.0 ms; 25k-cell helix (FP32, 7,205 rows)
-// 145 -> 91 ms; the 40k pipe's fused Jacobi cycle (FP32, 2,520 rows) 58.1 ->
-// 55.4 ms per 100 iterations.
+// TB/s.  Measured without and with it, the rest of the code the same: three
+// iterations of the wall-function loop on the 207k-cell helix (FP64, MCGS),
+// whose CF level of 8,530 rows with the 47 + 46 colours below it becomes one 582
+// MB product, 442 -> 287 ms; the 64^3 Poisson solve (1,073 rows, 44 colours)
+// 18.4 -> 9.7 ms; 25k-cell helix (FP32, 7,205 rows) 112 -> 72 ms; the 40k
+// pipe's fused Jacobi cycle (FP32, 2,443 rows) 52.1 -> 50.0 ms per 100
+// iterations; the 64k pipe's Chebyshev cycle (FP64) 33.0 -> 32.9 per 40.
+// Setting it up takes 115, 9, 48 and 1 ms.
 #pragma once
 
 #include <vector>

@@ -124,10 +124,9 @@ void GnnModel::refreshWeights(hipStream_t s) {
 // stream, and the first 16 MB through a new one cost 0.33 ms a MB in page
 // faults.  Large copies therefore go by the null stream, whose ring is in use
 // since the mesh was uploaded, behind the model's own work; that costs 5 us a
-// copy, which small ones do not win back.  Ten forward and gradient calls of a
-// new model: 16.8 and 11.6 -> 7.2 ms at 40,320 rows (the first alone 2.5 ->
-// 0.8), 18.6 -> 16.5 at 115,200 (6.5 -> 1.9); a later call 0.58 -> 0.59 and
-// 1.29 -> 1.30 ms.
+// copy, which small ones do not win back.  First forward and gradient call of
+// a new model: 2.0 -> 0.8 ms at 40,320 rows, 6.6 -> 2.1 ms at 115,200; a later
+// call 0.62 and 1.3 ms either way.
 const float* GnnModel::stage(const float* host, int width, DBuf<float>& d) {
   const std::size_t bytes = sizeof(float) * (std::size_t)n_ * width;
   if (bytes < kStageByNull) {

@@ -1691,9 +1691,9 @@ H8Solver::Bytes H8Solver::algorithmicBytes() const {
   const double n = nc_, nnz = (double)fineNnz_;
   // y = A x, FP64 values, int32 columns and row pointers, x and y once
   b.fineSpmv = nnz * (8 + 4) + (n + 1) * 4 + n * 8 + n * 8;
-  // refresh: row/diag pointers, per-nnz column + term offset + value write,
-  // per-term packed word, B table once, rAU once, diagonal write
-  b.refresh = (n + 1) * 4 + n * 4 + nnz * (4 + 4 + 8) + (double)F_.nzTerm.size() * 4 + n * 24 * 8 + nv_ * 8.0 + n * 8;
+  // refresh: row/diag pointers, per-nnz column + packed terms + value write,
+  // cell refs and B table once, rAU once, diagonal write
+  b.refresh = (n + 1) * 4 + n * 4 + nnz * (4 + 4 + 8) + n * (8 * 4 + 24 * 8) + nv_ * 8.0 + n * 8;
   // one forward sweep: A (values+cols), row pointers, b (3), diag, u read+write (3 each)
   b.momGsSweep = momNnz_ * 12.0 + (nv_ + 1) * 4.0 + nv_ * (24.0 + 8.0 + 48.0);
   b.convLocal = n * (8 * 4 + 9 * 8 + 8 + 64 * 8) + nv_ * 24.0;
