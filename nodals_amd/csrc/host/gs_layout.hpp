@@ -3,7 +3,9 @@
 #pragma once
 
 #include <algorithm>
+#include <exception>
 #include <numeric>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -75,14 +77,30 @@ GsLayout gsLayout(int ncolors, const std::vector<int>& off, const int* order, co
     const int cj = colorOf[(std::size_t)j];
     return half == GsHalf::all || (half == GsHalf::lower ? cj < c : cj > c);
   };
+  // body(colour, first row, rows) for every colour.  What a worker throws is
+  // thrown here after all have ended; slices that get no thread run here.
   auto eachColour = [&](auto&& body) {
     const int nt = std::max(1, std::min(ncolors, off.back() < 4096 ? 1 : hostThreads(0)));
-    std::vector<std::thread> pool;
-    for (int t = 0; t < nt; ++t)
-      pool.emplace_back([&, t]() {
+    std::vector<std::exception_ptr> error((std::size_t)nt);
+    auto slice = [&](int t) {
+      try {
         for (int c = t; c < ncolors; c += nt) body(c, off[(std::size_t)c], off[(std::size_t)c + 1] - off[(std::size_t)c]);
-      });
+      } catch (...) {
+        error[(std::size_t)t] = std::current_exception();
+      }
+    };
+    std::vector<std::thread> pool;
+    pool.reserve((std::size_t)nt);
+    int t = 1;
+    try {
+      for (; t < nt; ++t) pool.emplace_back(slice, t);
+    } catch (const std::system_error&) {
+    }
+    slice(0);
+    for (; t < nt; ++t) slice(t);
     for (std::thread& th : pool) th.join();
+    for (const std::exception_ptr& e : error)
+      if (e) std::rethrow_exception(e);
   };
   eachColour([&](int c, int b, int n) {
     if (n <= 0) return;

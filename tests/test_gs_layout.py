@@ -1,6 +1,11 @@
 """Storage of the multicolour Gauss-Seidel slots (csrc/host/gs_layout.hpp, no
 GPU): linear in the entries, also where a colour holds a few rows of thousands
 of entries beside thousands of short ones."""
+import resource
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import scipy.sparse as sp
 
@@ -47,3 +52,34 @@ def test_mesh_operator_storage():
     lower, upper, both = slots(A)
     off = A.nnz - A.shape[0]
     assert lower < 1.7 * off / 2 and upper < 1.7 * off / 2 and both < 1.3 * off
+
+
+LIMITED = """
+import resource, sys
+import numpy as np
+from nodals_amd._lib import System
+from tests.test_gs_layout import hub_system
+A = hub_system(12001, 2)
+S = System(A.indptr.astype(np.int64), A.indices.astype(np.int32), A.data, "terminal=100", device=False)
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + int(sys.argv[1]), resource.RLIM_INFINITY))
+try:
+    print(*S.get("gs_slots", 3, np.int64))
+except Exception as e:
+    print(type(e).__name__, e)
+"""
+
+
+def test_layout_without_room_for_threads():
+    """The workers' stacks (8 MB each) do not fit the address space: their
+    colours are laid out by the caller; without room for the layout either,
+    the call ends with an error, never the process."""
+    root = Path(__file__).resolve().parents[1]
+    out = []
+    for room in (7 << 20, 1 << 18):
+        r = subprocess.run([sys.executable, "-c", LIMITED, str(room)], cwd=root, capture_output=True, text=True,
+                           timeout=120, preexec_fn=lambda: resource.setrlimit(resource.RLIMIT_STACK, (8 << 20, 8 << 20)))
+        assert r.returncode == 0, r.stderr[-500:]
+        out.append(r.stdout.strip())
+    assert out[0] == " ".join(map(str, slots(hub_system(12001, 2))))
+    assert out[1] == out[0] or out[1].startswith(("NodalsError", "MemoryError"))
