@@ -169,7 +169,7 @@ struct WallConsts {
 //
 // LANES = 1: one thread a point, its samples and their fit in turn.  LANES =
 // 8: lane m of a point takes active sample m and the fit is shared (the same
-// results); taken for three or more points, where the one-thread chain of
+// steps); taken for three or more points, where the one-thread chain of
 // exponentials left one wavefront a SIMD busy: 375 us against 148 us for the
 // 23,040 five-point fits of the 40k pipe.
 template <int LANES>

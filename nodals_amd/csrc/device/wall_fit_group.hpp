@@ -4,9 +4,11 @@
 // Lane m of a group owns active sample m: its pointwise root, and its term of
 // every objective, gradient and Hessian evaluation.  The terms are then
 // gathered from the lanes and summed in sample order by the same
-// expressions, so all lanes of a group take the same branches and the
-// results are those of the one-thread fit.  The fit is a serial chain of
-// exponentials; five of its six evaluations a step run side by side here.
+// expressions, so all lanes of a group take the same branches and the search
+// takes the steps of the one-thread fit; what the compiler fuses may round
+// differently, which the golden section's branches can turn into its
+// resolution of 1e-5.  The fit is a serial chain of exponentials; five of its
+// six evaluations a step run side by side here.
 #pragma once
 
 #include "sst_physics.hpp"
